@@ -11,8 +11,10 @@
 // tiles of 256 x 256, and products that the tile kernel would run on few CUs or mostly empty
 // tiles (small_gemm_preferred's rate estimate), take the 64 x 64 small-product kernel (with K
 // split over the stream's workspace where its tiles alone would leave CUs idle:
-// small_gemm_splits); the rest (extents that split a 16-byte chunk) the staged kernel.  Unsigned bytes (lava_hip_gemm_u8_u32) take the same choice among the tile and small
-// kernels' unsigned forms, and a one-thread-per-element kernel where the staged kernel would run.
+// small_gemm_splits); operands that are not 16-byte aligned or whose extents split a 16-byte chunk
+// that kernel's any-alignment form; and the rest (rows shorter than 16 bytes) the staged kernel.
+// Unsigned bytes (lava_hip_gemm_u8_u32) take the same choice among the kernels' unsigned forms, and a
+// one-thread-per-element kernel where the staged kernel would run.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -82,6 +84,19 @@ int gemm_entry(const char* name, const void* A, const void* B, void* C, int64_t 
             return launch_gemm_mid<T, OutT, EPI, U8>(a, b, c, M, N, K, lda, ldb, ldc, s, epi, mfit == TN_RAGGED, arow,
                                                      !brow);
     }
+    // the 64 x 64 small-product kernel; any: its form for operands of any alignment and extent
+    auto run_small = [&](bool any) {
+        if constexpr (!EPI) {
+            const SmallSplit sp = pin == 2 ? SmallSplit{} : small_gemm_splits<T>(M, N, K);
+            // under graph capture, split only within the workspace the stream already has
+            if (sp.splits > 1 && small_splitk_bytes<T>(M, N, sp) <= stream_workspace_cap(stream))
+                return launch_gemm_small_splitk<T, U8>(a, b, c, M, N, K, lda, ldb, ldc, arow, brow, stream, sp, any);
+        }
+        if constexpr (U8)
+            return launch_gemm_small_u8(a, b, c, M, N, K, lda, ldb, ldc, arow, brow, s, any);
+        else
+            return launch_gemm_small<T, OutT, EPI>(a, b, c, M, N, K, lda, ldb, ldc, arow, brow, s, epi, any);
+    };
     bool use_small;
     if (pin == 2)
         use_small = small_fits;
@@ -89,24 +104,15 @@ int gemm_entry(const char* name, const void* A, const void* B, void* C, int64_t 
         use_small = false;
     else
         use_small = small_fits && small_gemm_preferred<T>(M, N, K);
-    if (use_small) {
-        if constexpr (!EPI) {
-            const SmallSplit sp = pin == 2 ? SmallSplit{} : small_gemm_splits<T>(M, N, K);
-            // under graph capture, split only within the workspace the stream already has
-            if (sp.splits > 1 && small_splitk_bytes<T>(M, N, sp) <= stream_workspace_cap(stream))
-                return launch_gemm_small_splitk<T, U8>(a, b, c, M, N, K, lda, ldb, ldc, arow, brow, stream, sp);
-        }
-        if constexpr (U8)
-            return launch_gemm_small_u8(a, b, c, M, N, K, lda, ldb, ldc, arow, brow, s);
-        else
-            return launch_gemm_small<T, OutT, EPI>(a, b, c, M, N, K, lda, ldb, ldc, arow, brow, s, epi);
-    }
+    if (use_small) return run_small(false);
     if (fit != TN_NO && pin != 3) {
         if constexpr (U8)
             return launch_gemm_tn_u8(a, b, c, M, N, K, lda, ldb, ldc, s, fit == TN_RAGGED, arow, !brow);
         else
             return launch_gemm_tn<T, OutT, EPI>(a, b, c, M, N, K, lda, ldb, ldc, s, epi, fit == TN_RAGGED, arow, !brow);
     }
+    // operands that split a 16-byte chunk or are not 16-byte aligned
+    if (pin != 3 && small_any_fits<T>(M, N, K, arow, brow)) return run_small(true);
     if constexpr (U8) {
         LAVA_REQUIRE((M * N + 255) / 256 <= 0x7fffffff, LAVA_HIP_ERR_UNSUPPORTED, "%s: problem too large", name);
         return launch_gemm_u8_generic(reinterpret_cast<const uint8_t*>(a), reinterpret_cast<const uint8_t*>(b),

@@ -4,8 +4,8 @@
 //    K-slice of 64 bytes staged through LDS with bounds-predicated loads, so it
 //    covers row- and column-major A and B and extents that are not tile
 //    multiples (the clamp-to-zero of a TENSOR_CLAMP_CONSTANT load,
-//    src/vocabulary/tensor.jl:46-51).  It is the fallback behind the fast TN
-//    kernel and the path for small problems.
+//    src/vocabulary/tensor.jl:46-51).  It takes what has no 16 bytes along a row (K, M or N
+//    below 8 sixteen-bit or 16 eight-bit elements).
 //  * gemm_small_kernel: the products too small to fill the chip with 256 x 256
 //    tiles (16 or fewer of them, e.g. the 256^3 fp16 configuration): 64 x 64 tiles,
 //    K in chunks of 512 bytes loaded with 16-byte loads, all in flight at once, the
@@ -101,6 +101,26 @@ __global__ void __launch_bounds__(256) gemm_staged_kernel(const T* __restrict__ 
         }
 }
 
+// 16 bytes from an address aligned to one byte: one global_load_dwordx4 (global memory takes
+// unaligned vector loads under the HSA ABI).
+__device__ __forceinline__ uint4 any_load(const void* p) {
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    typedef u32x4 u32x4_any __attribute__((aligned(1)));
+    const u32x4 v = *reinterpret_cast<const u32x4_any*>(p);
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+
+// x shifted down by `bits` (0 .. 128), zeros from above.
+__device__ __forceinline__ uint4 any_shift(uint4 x, int bits) {
+    const uint64_t l = (uint64_t)x.y << 32 | x.x, h = (uint64_t)x.w << 32 | x.z;
+    const bool far = bits >= 64;
+    const uint64_t lo = far ? h : l, hi = far ? 0u : h;
+    const int b = bits & 63;
+    uint64_t rl = b ? (lo >> b) | (hi << (64 - b)) : lo, rh = hi >> b;
+    if (bits >= 128) rl = rh = 0;
+    return make_uint4((uint32_t)rl, (uint32_t)(rl >> 32), (uint32_t)rh, (uint32_t)(rh >> 32));
+}
+
 // 64 x 64 C tile per workgroup of 4 wavefronts (32 x 32 each: 2 x 2 MFMA 16x16 tiles).  K runs
 // in chunks of 512 bytes.  A chunk of one operand is 64 rows (m or n) x 512 bytes = 2048 16-byte
 // loads, 8 per thread, all issued before any is waited for; the next chunk's loads are in flight
@@ -127,7 +147,16 @@ __global__ void __launch_bounds__(256) gemm_staged_kernel(const T* __restrict__ 
 // 128 (RA + CB) + 16384 Kp added, RA / CB the sums of its row's / column's flipped bytes over the
 // Kp k-values the workgroup multiplied (K padded to the 64-byte k-step: a padded byte reads 0,
 // flips to -128 in both operands, and its terms cancel), all modulo 2^32.
-template <typename T, bool AROW, bool BROW, typename OutT, bool EPI, bool U8 = false>
+// ANY: operands of any alignment, leading dimension and extent (a packed column-major array of odd
+// height has no two rows aligned alike).  A thread's 16 bytes are then one load of element
+// alignment, always whole and always inside the matrix: a chunk that would pass the end of its row
+// (K, M or N) is read from the row's last 16 bytes instead, a row past the last from the last row,
+// both from clamped addresses, so every load of a K chunk is in flight at once without a branch.  On
+// the way into LDS the pulled-back chunks are shifted down into place with zeros behind the end of
+// K (any_shift), only in workgroups and K chunks that reach an end.  Bound by the latency of a chunk's
+// loads, like the aligned form; fp16, all column-major, 1111 x 1333 x 777: 18.5 us a call (125
+// TFLOP/s) against 99.3 on the staged kernel, which loads element by element.
+template <typename T, bool AROW, bool BROW, typename OutT, bool EPI, bool U8 = false, bool ANY = false>
 __global__ void __launch_bounds__(256) gemm_small_kernel(const T* __restrict__ A, const T* __restrict__ B,
                                                          OutT* __restrict__ C, int64_t M, int64_t N, int64_t K,
                                                          int64_t lda, int64_t ldb, int64_t ldc, Epilogue epi,
@@ -165,6 +194,19 @@ __global__ void __launch_bounds__(256) gemm_small_kernel(const T* __restrict__ A
             const int e = tid + 256 * i;
             int64_t rr, kk;
             const T* p;
+            if constexpr (ANY) {
+                if constexpr (decltype(kcont)::value) {
+                    rr = min(r0 + (e >> 5), rows - 1);
+                    kk = min(k0 + (int64_t)EV * (e & 31), ke - EV);
+                    p = X + rr * ld + kk;
+                } else {
+                    kk = min(k0 + e / JR, ke - 1);
+                    rr = min(r0 + (int64_t)EV * (e % JR), rows - EV);
+                    p = X + kk * ld + rr;
+                }
+                reg[i] = any_load(p);
+                continue;
+            }
             if constexpr (decltype(kcont)::value) {
                 rr = r0 + (e >> 5);
                 kk = k0 + (int64_t)EV * (e & 31);
@@ -178,11 +220,23 @@ __global__ void __launch_bounds__(256) gemm_small_kernel(const T* __restrict__ A
             if (rr < rows && kk < ke) reg[i] = *reinterpret_cast<const uint4*>(p);
         }
     };
-    auto store = [&](uint8_t* S, auto kcont, auto tr, const uint4* reg) {
+    auto store = [&](uint8_t* S, auto kcont, auto tr, const uint4* reg, int64_t r0, int64_t rows, int64_t k0) {
+        // ANY: this thread's chunks all start at the same place of their row, so one shift serves them
+        const bool k_end = k0 + KC > ke, r_end = r0 + 64 > rows;   // uniform
+        int shift = 0;
+        if constexpr (ANY) {
+            const int64_t over = decltype(kcont)::value ? k0 + (int64_t)EV * (tid & 31) + EV - ke
+                                                        : r0 + (int64_t)EV * (tid % JR) + EV - rows;
+            shift = (int)max((int64_t)0, min(over, (int64_t)EV));
+        }
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const int e = tid + 256 * i;
             uint4 x = reg[i];
+            if constexpr (ANY) {
+                if (decltype(kcont)::value ? k_end : r_end) x = any_shift(x, shift * 8 * (int)sizeof(T));
+                if (!decltype(kcont)::value && k_end && k0 + e / JR >= ke) x = make_uint4(0, 0, 0, 0);
+            }
             if constexpr (U8) {
                 x.x ^= 0x80808080u;
                 x.y ^= 0x80808080u;
@@ -254,8 +308,8 @@ __global__ void __launch_bounds__(256) gemm_small_kernel(const T* __restrict__ A
     load(A, AK{}, lda, m0, M, kb, ra);
     load(B, BK{}, ldb, n0, N, kb, rb);
     for (int64_t k0 = kb; k0 < ke; k0 += KC) {
-        store(As, AK{}, ATR{}, ra);
-        store(Bs, BK{}, BTR{}, rb);
+        store(As, AK{}, ATR{}, ra, m0, M, k0);
+        store(Bs, BK{}, BTR{}, rb, n0, N, k0);
         __syncthreads();
         if (k0 + KC < ke) {   // the next chunk, in flight during this one's MFMAs
             load(A, AK{}, lda, m0, M, k0 + KC, ra);
@@ -435,8 +489,18 @@ bool small_gemm_fits(const void* A, const void* B, int64_t M, int64_t N, int64_t
     return aligned(A, 16) && aligned(B, 16) && lda % EV == 0 && ldb % EV == 0 &&
            ((arow || !brow) ? K % EV == 0 : true) && (arow || M % EV == 0) && (!brow || N % EV == 0);
 }
+// The ANY form reads 16 bytes inside each row, so the contiguous extent of each operand holds at
+// least that much; nothing else is asked of it.  It leads the staged kernel wherever it fits (99.3 ->
+// 18.5 us at 1111 x 1333 x 777); the aligned forms lead it, so it runs where none of them fits.
+template <typename T>
+bool small_any_fits(int64_t M, int64_t N, int64_t K, bool arow, bool brow) {
+    constexpr int64_t EV = 16 / (int64_t)sizeof(T);
+    if ((M + 63) / 64 > 65535 || (N + 63) / 64 > 0x7fffffff) return false;
+    return ((arow || !brow) ? K >= EV : K > 0) && (arow || M >= EV) && (!brow || N >= EV);
+}
 #define LAVA_SMALL_RULE_INST(T)                                                                                      \
     template bool small_gemm_preferred<T>(int64_t, int64_t, int64_t);                                           \
+    template bool small_any_fits<T>(int64_t, int64_t, int64_t, bool, bool);                                     \
     template bool small_gemm_fits<T>(const void*, const void*, int64_t, int64_t, int64_t, int64_t, int64_t, bool, bool);
 LAVA_SMALL_RULE_INST(f16)
 LAVA_SMALL_RULE_INST(bf16)
@@ -447,35 +511,42 @@ namespace {
 template <typename T, typename OutT, bool EPI, bool U8 = false>
 int launch_small_grid(const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
                       int64_t ldc, bool arow, bool brow, hipStream_t s, const Epilogue& epi, int splits,
-                      int64_t kspan, int64_t zstride) {
+                      int64_t kspan, int64_t zstride, bool any) {
     const dim3 grid((unsigned)((N + 63) / 64), (unsigned)((M + 63) / 64), (unsigned)splits);
-    if (arow && brow)
-        hipLaunchKernelGGL((gemm_small_kernel<T, true, true, OutT, EPI, U8>), grid, dim3(256), 0, s, A, B, C, M, N, K,
-                           lda, ldb, ldc, epi, kspan, zstride);
-    else if (arow)
-        hipLaunchKernelGGL((gemm_small_kernel<T, true, false, OutT, EPI, U8>), grid, dim3(256), 0, s, A, B, C, M, N, K,
-                           lda, ldb, ldc, epi, kspan, zstride);
-    else if (brow)
-        hipLaunchKernelGGL((gemm_small_kernel<T, false, true, OutT, EPI, U8>), grid, dim3(256), 0, s, A, B, C, M, N, K,
-                           lda, ldb, ldc, epi, kspan, zstride);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, A, B, C, M, N, K, lda, ldb, ldc, epi, kspan, zstride);
+    };
+    auto by_layout = [&](auto anytag) {
+        constexpr bool ANY = decltype(anytag)::value;
+        if (arow && brow)
+            go(gemm_small_kernel<T, true, true, OutT, EPI, U8, ANY>);
+        else if (arow)
+            go(gemm_small_kernel<T, true, false, OutT, EPI, U8, ANY>);
+        else if (brow)
+            go(gemm_small_kernel<T, false, true, OutT, EPI, U8, ANY>);
+        else
+            go(gemm_small_kernel<T, false, false, OutT, EPI, U8, ANY>);
+    };
+    if (any)
+        by_layout(std::integral_constant<bool, true>{});
     else
-        hipLaunchKernelGGL((gemm_small_kernel<T, false, false, OutT, EPI, U8>), grid, dim3(256), 0, s, A, B, C, M, N,
-                           K, lda, ldb, ldc, epi, kspan, zstride);
-    LAVA_LAUNCH_CHECK(U8 ? "gemm_small_kernel<u8>" : "gemm_small_kernel");
+        by_layout(std::integral_constant<bool, false>{});
+    LAVA_LAUNCH_CHECK(any ? (U8 ? "gemm_small_kernel<u8,any>" : "gemm_small_kernel<any>")
+                          : (U8 ? "gemm_small_kernel<u8>" : "gemm_small_kernel"));
     return LAVA_HIP_OK;
 }
 }  // namespace
 
 int launch_gemm_small_u8(const int8_t* A, const int8_t* B, int32_t* C, int64_t M, int64_t N, int64_t K, int64_t lda,
-                         int64_t ldb, int64_t ldc, bool arow, bool brow, hipStream_t s) {
+                         int64_t ldb, int64_t ldc, bool arow, bool brow, hipStream_t s, bool any) {
     return launch_small_grid<int8_t, int32_t, false, true>(A, B, C, M, N, K, lda, ldb, ldc, arow, brow, s, Epilogue{},
-                                                           1, K > 0 ? K : 1, 0);
+                                                           1, K > 0 ? K : 1, 0, any);
 }
 
 template <typename T, typename OutT, bool EPI>
 int launch_gemm_small(const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
-                      int64_t ldc, bool arow, bool brow, hipStream_t s, const Epilogue& epi) {
-    return launch_small_grid<T, OutT, EPI>(A, B, C, M, N, K, lda, ldb, ldc, arow, brow, s, epi, 1, K > 0 ? K : 1, 0);
+                      int64_t ldc, bool arow, bool brow, hipStream_t s, const Epilogue& epi, bool any) {
+    return launch_small_grid<T, OutT, EPI>(A, B, C, M, N, K, lda, ldb, ldc, arow, brow, s, epi, 1, K > 0 ? K : 1, 0, any);
 }
 
 template <typename T>
@@ -508,7 +579,7 @@ template size_t small_splitk_bytes<int8_t>(int64_t, int64_t, const SmallSplit&);
 template <typename T, bool U8>
 int launch_gemm_small_splitk(const T* A, const T* B, typename Mfma16<T>::acc_elem* C, int64_t M, int64_t N, int64_t K,
                              int64_t lda, int64_t ldb, int64_t ldc, bool arow, bool brow, void* stream,
-                             const SmallSplit& sp) {
+                             const SmallSplit& sp, bool any) {
     using Acc = typename Mfma16<T>::acc_elem;
     hipStream_t s = as_stream(stream);
     return with_stream_workspace(small_splitk_bytes<T>(M, N, sp), stream, [&](void* ws) {
@@ -516,7 +587,7 @@ int launch_gemm_small_splitk(const T* A, const T* B, typename Mfma16<T>::acc_ele
         // unsigned: each split's partial carries its own correction, so the wrapped sum of the
         // partials is the product
         int rc = launch_small_grid<T, Acc, false, U8>(A, B, P, M, N, K, lda, ldb, N, arow, brow, s, Epilogue{},
-                                                     sp.splits, sp.kspan, M * N);
+                                                     sp.splits, sp.kspan, M * N, any);
         if (rc != LAVA_HIP_OK) return rc;
         if (N % 4 == 0)
             hipLaunchKernelGGL((splitk_sum_kernel<Acc, 4>), dim3((unsigned)((N + 1023) / 1024), (unsigned)M), dim3(256),
@@ -532,19 +603,19 @@ template SmallSplit small_gemm_splits<f16>(int64_t, int64_t, int64_t);
 template SmallSplit small_gemm_splits<bf16>(int64_t, int64_t, int64_t);
 template SmallSplit small_gemm_splits<int8_t>(int64_t, int64_t, int64_t);
 template int launch_gemm_small_splitk<f16, false>(const f16*, const f16*, float*, int64_t, int64_t, int64_t, int64_t,
-                                                  int64_t, int64_t, bool, bool, void*, const SmallSplit&);
+                                                  int64_t, int64_t, bool, bool, void*, const SmallSplit&, bool);
 template int launch_gemm_small_splitk<bf16, false>(const bf16*, const bf16*, float*, int64_t, int64_t, int64_t,
-                                                   int64_t, int64_t, int64_t, bool, bool, void*, const SmallSplit&);
+                                                   int64_t, int64_t, int64_t, bool, bool, void*, const SmallSplit&, bool);
 template int launch_gemm_small_splitk<int8_t, false>(const int8_t*, const int8_t*, int32_t*, int64_t, int64_t, int64_t,
-                                                     int64_t, int64_t, int64_t, bool, bool, void*, const SmallSplit&);
+                                                     int64_t, int64_t, int64_t, bool, bool, void*, const SmallSplit&, bool);
 template int launch_gemm_small_splitk<int8_t, true>(const int8_t*, const int8_t*, int32_t*, int64_t, int64_t, int64_t,
-                                                    int64_t, int64_t, int64_t, bool, bool, void*, const SmallSplit&);
+                                                    int64_t, int64_t, int64_t, bool, bool, void*, const SmallSplit&, bool);
 
 #define LAVA_STAGED_INST(T, O, E)                                                                              \
     template int launch_gemm_staged<T, O, E>(const T*, const T*, O*, int64_t, int64_t, int64_t, int64_t, int64_t, \
                                              int64_t, bool, bool, hipStream_t, const Epilogue&);                  \
     template int launch_gemm_small<T, O, E>(const T*, const T*, O*, int64_t, int64_t, int64_t, int64_t, int64_t,  \
-                                            int64_t, bool, bool, hipStream_t, const Epilogue&);
+                                            int64_t, bool, bool, hipStream_t, const Epilogue&, bool);
 LAVA_STAGED_INST(f16, float, false)
 LAVA_STAGED_INST(bf16, float, false)
 LAVA_STAGED_INST(int8_t, int32_t, false)

@@ -23,9 +23,13 @@ bool small_gemm_preferred(int64_t M, int64_t N, int64_t K);
 template <typename T>
 bool small_gemm_fits(const void* A, const void* B, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, bool arow,
                      bool brow);
+// The kernel's ANY form (any alignment, leading dimension and extent; `any` of the launchers below):
+// whether every row it reads along holds a 16-byte chunk.
+template <typename T>
+bool small_any_fits(int64_t M, int64_t N, int64_t K, bool arow, bool brow);
 template <typename T, typename OutT, bool EPI>
 int launch_gemm_small(const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
-                      int64_t ldc, bool arow, bool brow, hipStream_t s, const Epilogue& epi);
+                      int64_t ldc, bool arow, bool brow, hipStream_t s, const Epilogue& epi, bool any);
 
 // Split K for the small kernel's plain products (no epilogue): a product of at most 256 64 x 64
 // tiles and at least 8 K chunks of 512 bytes (16 above 128 tiles) runs in `splits` K ranges of kspan elements (each
@@ -45,10 +49,10 @@ size_t small_splitk_bytes(int64_t M, int64_t N, const SmallSplit& sp);
 template <typename T, bool U8 = false>
 int launch_gemm_small_splitk(const T* A, const T* B, typename Mfma16<T>::acc_elem* C, int64_t M, int64_t N, int64_t K,
                              int64_t lda, int64_t ldb, int64_t ldc, bool arow, bool brow, void* stream,
-                             const SmallSplit& sp);
+                             const SmallSplit& sp, bool any);
 // Unsigned bytes on the small kernel, unsplit (flipped bytes, signed MFMAs, row / column sums).
 int launch_gemm_small_u8(const int8_t* A, const int8_t* B, int32_t* C, int64_t M, int64_t N, int64_t K, int64_t lda,
-                         int64_t ldb, int64_t ldc, bool arow, bool brow, hipStream_t s);
+                         int64_t ldb, int64_t ldc, bool arow, bool brow, hipStream_t s, bool any);
 
 // The 16x16x16 vocabulary-tile GEMM (fp16 -> fp32); M, N, K multiples of 16.
 int launch_coopmat_tiles(const f16* A, const f16* B, float* C, int64_t M, int64_t N, int64_t K, int64_t lda,
