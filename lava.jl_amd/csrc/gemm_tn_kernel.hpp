@@ -233,7 +233,8 @@ struct TnSide<T, false, 128> {
     // fragment t (columns 16 t of the half) of k-step u (32 rows of K): two transposing reads, k rows
     // 8 g + [0, 4) and 8 g + [4, 8) of the k-step
     __device__ __forceinline__ uint4 read16(const uint8_t* slice, int u, int t) const {
-        const uint8_t* b = slice + u * 32 * 256 + mr16 + c16[t];
+        // (blocks 4 to 7 are the other half's: their chunks differ in the slot's top bit)
+        const uint8_t* b = slice + u * 32 * 256 + mr16 + (t < 4 ? c16[t & 3] : c16[t & 3] ^ 128);
         const tn_s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
             (__attribute__((address_space(3))) tn_s16x4*)(const __attribute__((address_space(3))) uint8_t*)b);
         const tn_s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(

@@ -33,6 +33,7 @@
 #include <type_traits>
 #include <vector>
 
+#include "gemm_w8a16.hpp"
 #include "lava_coopmat.hpp"
 #include "lava_hip_internal.hpp"
 #include "lds_dma.hpp"
@@ -298,20 +299,6 @@ struct KmCfg {
     static_assert(BUFS * STAGE >= MB * KM_TILES * 64 * 16, "the K-range sums reuse a wavefront's ring");
 };
 
-// 8 int8 weights (two dwords, k ascending) -> the 8 fp16 values of a B operand
-__device__ __forceinline__ f16x8 km_dequant(uint32_t lo, uint32_t hi) {
-    const uint32_t x0 = lo ^ 0x80808080u, x1 = hi ^ 0x80808080u;
-    // bytes 0-3 of the selector's source pair are the 0x64 register, 4-7 the weights
-    uint4 v;
-    v.x = __builtin_amdgcn_perm(x0, 0x64646464u, 0x00050004u);
-    v.y = __builtin_amdgcn_perm(x0, 0x64646464u, 0x00070006u);
-    v.z = __builtin_amdgcn_perm(x1, 0x64646464u, 0x00050004u);
-    v.w = __builtin_amdgcn_perm(x1, 0x64646464u, 0x00070006u);
-    const f16x8 bias = {(f16)-1152.f, (f16)-1152.f, (f16)-1152.f, (f16)-1152.f,
-                        (f16)-1152.f, (f16)-1152.f, (f16)-1152.f, (f16)-1152.f};
-    return __builtin_bit_cast(f16x8, v) + bias;   // exact: w = (1152 + w) - 1152
-}
-
 // X column-major: the stage's X is [128 k-lines][16 rows] (32-byte lines), line L stored at
 // km_xline(L) -- lines 16 apart would share banks in a fragment read, the permutation moves every
 // other group of 16 to the other half of the banks -- and read with ds_read_b64_tr_b16: source
@@ -454,7 +441,7 @@ __global__ void __launch_bounds__(64 * KM_WAVES) w8a16_kmajor_kernel(const f16* 
         for (int h = 0; h < 2; ++h)
 #pragma unroll
             for (int t = 0; t < KM_TILES; ++t) {
-                const f16x8 w0 = km_dequant(wf[h][t].x, wf[h][t].y), w1 = km_dequant(wf[h][t].z, wf[h][t].w);
+                const f16x8 w0 = w8_dequant(wf[h][t].x, wf[h][t].y), w1 = w8_dequant(wf[h][t].z, wf[h][t].w);
 #pragma unroll
                 for (int b = 0; b < MB; ++b) {
                     acc[b][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[b][h][0], w0, acc[b][t], 0, 0, 0);
@@ -544,6 +531,7 @@ struct W8Plan {
     bool x_copy = false;
     int splits = 1;
     int mb = 1;                  // W8_KMAJOR: 16-row blocks of X per workgroup
+    int bn = 0;                  // W8_KMAJOR: the tiled kernel's columns per tile (0: the streaming kernel)
     int ksteps = 0;              // the per-wavefront step count of an unrolled instance, or 0
     // split-K workspace (W8_SPLIT with splits > 1): the arrival counters (one per column and
     // row block, zero between calls) in the first counter_bytes, then the partial blocks
@@ -585,6 +573,18 @@ static W8Plan plan_w8a16(const void* X, const void* W, int64_t M, int64_t N, int
         p.mb = M <= 16 ? 1 : (M <= 32 ? 2 : 4);
         while (p.mb > 1 && p.xrow && 32 * p.mb * p.kldx >= (int64_t(1) << 32)) p.mb /= 2;
         p.mblocks = (M + 16 * p.mb - 1) / (16 * p.mb);
+        // Batches: the tiled kernel once the streaming one would need more than 256 workgroups (a
+        // second one per CU), measured at K = 4096 (us, streaming / tiled): 72 x 5120 20.4 / 19.2, 192
+        // x 3072 22.6 / 19.8, 128 x 8192 25.3 / 20.1, 256 x 14336 89.0 / 33.4, but 128 x 4096 (256
+        // workgroups) 17.0 / 20.1 and 256 x 2048 16.7 / 19.6.  At most 64 rows stay a weight stream
+        // (one workgroup per 32 columns, 64 x 14336 23.9 / 20.6).  The tile is 128 x 64 or 128 x 128 by
+        // the time of its rounds over the 256 CUs, about 0.55 and 0.85 us per 128 k each: 256 x 8192
+        // (256 and 128 tiles) 27.1 / 31.6, 256 x 11008 (344 and 172) 41.5 / 33.3.
+        if (M > 64 && p.cblocks * p.mblocks > 256 && w8a16_batch_fits(M, N, p.kldx, K, ldw, p.xrow)) {
+            const int64_t mt = (M + 127) / 128;
+            const int64_t rounds64 = (mt * ((N + 63) / 64) + 255) / 256, rounds128 = (mt * ((N + 127) / 128) + 255) / 256;
+            p.bn = 11 * rounds64 > 17 * rounds128 ? 128 : 64;
+        }
         if (!x_ok) {
             p.x_copy = true;
             p.counter_bytes = W8_COUNTER_BYTES;
@@ -668,6 +668,9 @@ static int launch_w8a16(const W8Plan& p, const void* X, const void* W, const voi
             LAVA_LAUNCH_CHECK("w8a16_x_rows_kernel");
             xk = xr;
         }
+        if (p.bn)
+            return launch_w8a16_batch(xk, (const int8_t*)W, (const f16*)scale, (float*)Y, M, N, K, p.kldx, ldw, ldy, p.xrow,
+                                      p.yrow, p.bn, s);
         auto go = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3((unsigned)p.cblocks, (unsigned)p.mblocks), dim3(64 * KM_WAVES), 0, s, xk,
                                (const int8_t*)W, (const f16*)scale, (float*)Y, (int)M, (int)N, (int)K, p.kldx, ldw,
