@@ -32,6 +32,8 @@
 //    across groups of the XCD's heads (fa_order).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <cmath>
 #include <type_traits>
 #include <utility>
 
@@ -512,8 +514,10 @@ __global__ void __launch_bounds__(64 * F3_WAVES, 1) flash_fwd3_kernel(FaParams p
 // score wavefronts, also issue every K and V load and sum the rows of P (from the
 // fp16 fragments they read, in fp32) -- the score wavefront does only the scores and
 // the softmax.
+// QH = 1 gives each pair one 32-query half (128 queries per workgroup): a fragment then feeds one MFMA
+// and a key block takes 0.70 of the time for half the queries, for grids that 256-query workgroups
+// leave uneven or short of the 256 CUs (fa_narrow_preferred).
 constexpr int F5_PAIRS = 4;
-constexpr int F5_BQ = 64 * F5_PAIRS;   // 256 queries per workgroup
 constexpr int F5_BK = 64;
 constexpr int F5_KST = 3, F5_VST = 2;
 constexpr int F5_PFK = 4;              // K fragments read ahead of the MFMA that uses them
@@ -558,9 +562,11 @@ __device__ __forceinline__ void fa_scale_f16(f16x8& q, float c) {
 // and Q are staged 128 wide whatever DE is (the chunks past D are DMA-ed as zeros, so the LDS
 // layout, its swizzles and the DMA map stay those of D = 128); a smaller DE only drops the S^T
 // k-steps and the O^T row tiles that would multiply those zero columns.
-template <bool CAUSAL, int DE>
+template <bool CAUSAL, int DE, int QH>
 __global__ void __launch_bounds__(128 * F5_PAIRS, 1) flash_fwd5_kernel(FaParams p) {
     static_assert(DE == 64 || DE == 96 || DE == 128, "the MFMAs cover 64, 96 or 128 of the head dimension");
+    constexpr int PQ = 32 * QH;                // queries per pair
+    constexpr int BQ = PQ * F5_PAIRS;          // queries per workgroup
     constexpr int DH = 128;                    // staged width
     constexpr int RB = DH * 2;                 // 256 bytes per K / V row
     constexpr int CH = RB / 16;                // 16 chunks
@@ -570,30 +576,33 @@ __global__ void __launch_bounds__(128 * F5_PAIRS, 1) flash_fwd5_kernel(FaParams 
     constexpr int NSF = 2 * NKS;               // K fragments per block: (ks, kt)
     constexpr int NVF = 4 * NDT;               // V fragments per block: (key step kk, dt)
     constexpr int DPT = TILE / (1024 * F5_PAIRS);   // 4 DMA instructions per wavefront per tile
-    constexpr int PBUF = 8 * 1024;             // one pair's P^T fragments for one block
+    constexpr int PBUF = QH * 4 * 1024;             // one pair's P^T fragments for one block
     static_assert(DPT == 4, "4 DMA instructions per tile and wavefront");
     __shared__ __attribute__((aligned(1024))) uint8_t kbuf[F5_KST][TILE];   // [key][RB], chunk ^ key % 16
     __shared__ __attribute__((aligned(1024))) uint8_t vbuf[F5_VST][TILE];   // [key][RB], chunk ^ 4 (key % 4)
     __shared__ __attribute__((aligned(1024))) uint8_t pbuf[2][F5_PAIRS][PBUF];
-    __shared__ float abuf[2][F5_PAIRS][64];    // rescale factor per query of the next block
+    __shared__ float abuf[2][F5_PAIRS][PQ];    // rescale factor per query of the next block
     __shared__ int fbuf[2][F5_PAIRS];          // whether that block rescales
+    // Q on its way in, O on its way out, 32 rows of 256 bytes at xst[qh]: two halves use the pair's P
+    // buffers; one half's would not hold them, so it has room of its own
+    __shared__ __attribute__((aligned(1024))) uint8_t xbuf[QH == 1 ? F5_PAIRS : 1][QH == 1 ? 32 * RB : 16];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const bool is_s = w < F5_PAIRS;
-    const int pr = w & (F5_PAIRS - 1);         // the pair: queries q0 .. q0 + 63
-    const int nqb = (p.S + F5_BQ - 1) / F5_BQ;
+    const int pr = w & (F5_PAIRS - 1);         // the pair: queries q0 .. q0 + PQ - 1
+    const int nqb = (p.S + BQ - 1) / BQ;
     const int nbh = p.H * p.B;
     int bh, qb;
     fa_order(nqb, nbh, CAUSAL, bh, qb);
     const int hh = bh % p.H, bb = bh / p.H;
     const int64_t head = (int64_t)hh * p.sh + (int64_t)bb * p.sb;
     f16* Ob = p.O + (int64_t)hh * p.osh + (int64_t)bb * p.osb;
-    const int q0 = qb * F5_BQ + pr * 64;
+    const int q0 = qb * BQ + pr * PQ;
     const int r32 = lane & 31, h = lane >> 5;
     const int nkb_s = (p.S + F5_BK - 1) / F5_BK;
-    const int nkb = CAUSAL ? min((qb + 1) * (F5_BQ / F5_BK), nkb_s) : nkb_s;
-    const int last = CAUSAL ? min(nkb - 1, (q0 + 63) / F5_BK) : nkb - 1;   // this pair's last key block
+    const int nkb = CAUSAL ? min((qb + 1) * (BQ / F5_BK), nkb_s) : nkb_s;
+    const int last = CAUSAL ? min(nkb - 1, (q0 + PQ - 1) / F5_BK) : nkb - 1;   // this pair's last key block
 
     // LDS-DMA of K and V (issued by the output wavefronts): wavefront pr moves rows
     // 16 pr + 4 i + lane / 16 of a tile, physical chunk lane % 16 (K chunk ^ key % 16, V
@@ -633,8 +642,12 @@ __global__ void __launch_bounds__(128 * F5_PAIRS, 1) flash_fwd5_kernel(FaParams 
     // P^T fragment (kt, ks, qh) of pair pr in buffer b: 1 KB, lane l at 16 l
     const uint32_t p_lane = lds_addr(&pbuf[0][0][0]) + (uint32_t)pr * PBUF + 16u * lane;
     auto paddr = [&](int b, int kt, int ks, int qh) __attribute__((always_inline)) -> uint32_t {
-        return p_lane + (uint32_t)(b * F5_PAIRS * PBUF + ((kt * 2 + ks) * 2 + qh) * 1024);
+        return p_lane + (uint32_t)(b * F5_PAIRS * PBUF + ((kt * 2 + ks) * QH + qh) * 1024);
     };
+
+    uint32_t xst[QH];
+#pragma unroll
+    for (int qh = 0; qh < QH; ++qh) xst[qh] = QH == 1 ? lds_addr(&xbuf[pr][0]) : lds_addr(&pbuf[qh][pr][0]);
 
     // prologue DMAs (output wavefronts): K_0, K_1, K_2, V_0
     if (!is_s) {
@@ -645,31 +658,30 @@ __global__ void __launch_bounds__(128 * F5_PAIRS, 1) flash_fwd5_kernel(FaParams 
 
     if (is_s) {
         // ================= score wavefront =================
-        // The pair's 64 Q rows go to LDS first (this pair's P buffers, free until the first
-        // block's P is written), in the K tile's layout -- LDS-DMA of 4 whole rows per
+        // The pair's Q rows go to LDS first (two halves: this pair's P buffers, free until the
+        // first block's P is written), in the K tile's layout -- LDS-DMA of 4 whole rows per
         // instruction, chunk ^ row % 16, rows at or past S read zero -- and the Q^T
         // fragments are read from there: whole-row reads instead of 32 rows x 32 bytes per
         // load instruction.
-        const uint32_t qst[2] = {lds_addr(&pbuf[0][pr][0]), lds_addr(&pbuf[1][pr][0])};
         {
-            const uint32_t rows = (uint32_t)max(0, min(64, p.S - q0));
+            const uint32_t rows = (uint32_t)max(0, min(PQ, p.S - q0));
             const v4i rs = make_rsrc(p.Q + head + (int64_t)q0 * p.sl, rows * row_bytes);
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
+            for (int i = 0; i < 8 * QH; ++i) {
                 const int row = 4 * i + lane / CH;
                 const uint32_t v = chunk_ofs(row, (lane % CH) ^ (row & 15));
-                dma16(rs, v, 0u, __builtin_amdgcn_readfirstlane(qst[i / 8] + (uint32_t)((4 * i) % 32) * RB));
+                dma16(rs, v, 0u, __builtin_amdgcn_readfirstlane(xst[i / 8] + (uint32_t)((4 * i) % 32) * RB));
             }
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        f16x8 qf[2][NKS];   // Q^T B operands: query q0 + 32 qh + r32, d = 16 ks + 8 h + [0, 8)
+        f16x8 qf[QH][NKS];   // Q^T B operands: query q0 + 32 qh + r32, d = 16 ks + 8 h + [0, 8)
 #pragma unroll
-        for (int qh = 0; qh < 2; ++qh)
+        for (int qh = 0; qh < QH; ++qh)
 #pragma unroll
             for (int ks = 0; ks < NKS; ++ks)
-                qf[qh][ks] = *(const lds_f16x8*)(uintptr_t)(qst[qh] + (uint32_t)(r32 * RB + (((2 * ks + h) ^ (r32 & 15)) << 4)));
+                qf[qh][ks] = *(const lds_f16x8*)(uintptr_t)(xst[qh] + (uint32_t)(r32 * RB + (((2 * ks + h) ^ (r32 & 15)) << 4)));
 #pragma unroll
-        for (int qh = 0; qh < 2; ++qh)
+        for (int qh = 0; qh < QH; ++qh)
 #pragma unroll
             for (int ks = 0; ks < NKS; ++ks) {
                 const uint4 u = __builtin_bit_cast(uint4, qf[qh][ks]);
@@ -686,21 +698,21 @@ __global__ void __launch_bounds__(128 * F5_PAIRS, 1) flash_fwd5_kernel(FaParams 
         bool fast = c <= 1.f;                    // wavefront-uniform
         if (fast) {
 #pragma unroll
-            for (int qh = 0; qh < 2; ++qh)
+            for (int qh = 0; qh < QH; ++qh)
 #pragma unroll
                 for (int ks = 0; ks < NKS; ++ks) fa_scale_f16(qf[qh][ks], c);
         }
         const float c_raw = fast ? 1.f : c;      // the multiplier S needs on the fp32 path
         f16x8 ones{};                            // bias A operand: 1 at k = 0 of every key row
         ones[0] = h == 0 ? (f16)1.f : (f16)0.f;
-        f16x8 qm[2] = {f16x8{}, f16x8{}};         // bias B operand: -m at k = 0 of each query
+        f16x8 qm[QH] = {};                       // bias B operand: -m at k = 0 of each query
         // K fragment (kt, ks): row 32 kt + r32, chunk (2 ks + h) ^ (r32 % 16)
         uint32_t kb0[NKS];
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks)
             kb0[ks] = lds_addr(&kbuf[0][0]) + (uint32_t)(r32 * RB + (((2 * ks + h) ^ (r32 & 15)) << 4));
-        f32x16 st[2][2];           // st[kt][qh] register r: key 32 kt + 8 (r / 4) + 4 h + r % 4
-        float m_run[2] = {0.f, 0.f};
+        f32x16 st[2][QH];          // st[kt][qh] register r: key 32 kt + 8 (r / 4) + 4 h + r % 4
+        float m_run[QH] = {};
 
         // S_kb = K_kb Q^T (minus m), the softmax, P^T and the rescale factors into buffer b
         auto block = [&](int kb, int b, bool first) __attribute__((always_inline)) {
@@ -721,31 +733,32 @@ __global__ void __launch_bounds__(128 * F5_PAIRS, 1) flash_fwd5_kernel(FaParams 
 #pragma unroll
             for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-                for (int qh = 0; qh < 2; ++qh)
+                for (int qh = 0; qh < QH; ++qh)
                     st[kt][qh] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ones, qm[qh], f32x16{}, 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int i = 0; i < 2 * NSF; ++i) {   // MFMA i: fragment f = i / 2 (ks = f / 2, kt = f % 2), qh = i % 2
-                const int f = i >> 1, qh = i & 1, ks = f >> 1, kt = f & 1;
+            for (int i = 0; i < QH * NSF; ++i) {   // MFMA i: fragment f = i / QH (ks = f / 2, kt = f % 2), qh = i % QH
+                const int f = i / QH, qh = i % QH, ks = f >> 1, kt = f & 1;
                 st[kt][qh] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fr[f % F5_PFK], qf[qh][ks], st[kt][qh], 0, 0, 0);
-                if (qh == 1 && f + F5_PFK < NSF) fr[f % F5_PFK] = kread(f + F5_PFK);
+                if (qh == QH - 1 && f + F5_PFK < NSF) fr[f % F5_PFK] = kread(f + F5_PFK);
                 __builtin_amdgcn_sched_barrier(0);
             }
             // mask: causal key > query; else keys >= S.  A pair's causal last block is its diagonal
             // block (it starts at the pair's first query, kb * 64 = q0, for every pair with a query
             // below S; the others are never stored), where key tile 1 lies wholly above query half
             // 0 and key tile 0 wholly below query half 1: only the two diagonal 32 x 32 tiles compare.
+            // (A pair of one half starts at the block's first or 32nd key: every tile compares.)
             if (CAUSAL ? kb == last : (kb + 1) * F5_BK > p.S) {
-                int dv = CAUSAL ? 4 * h - r32 : kb * F5_BK + 4 * h - p.S;
+                int dv = CAUSAL ? 4 * h - r32 - (QH == 1 ? q0 & 32 : 0) : kb * F5_BK + 4 * h - p.S;
                 asm volatile("; mask" : "+v"(dv));
 #pragma unroll
                 for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-                    for (int qh = 0; qh < 2; ++qh)
+                    for (int qh = 0; qh < QH; ++qh)
 #pragma unroll
                         for (int r = 0; r < 16; ++r) {
                             const int kr = 32 * kt + 8 * (r >> 2) + (r & 3);
-                            if (CAUSAL && kt != qh) {
+                            if (QH == 2 && CAUSAL && kt != qh) {
                                 if (kt > qh) st[kt][qh][r] = -INFINITY;
                                 continue;
                             }
@@ -755,9 +768,9 @@ __global__ void __launch_bounds__(128 * F5_PAIRS, 1) flash_fwd5_kernel(FaParams 
             }
             // t = how far this block's largest exponent lies above the running maximum
             const bool fast_blk = fast;           // st holds S' (fast) or S (fp32 path)
-            float vl[2];   // this lane's largest score per query half
+            float vl[QH];   // this lane's largest score per query half
 #pragma unroll
-            for (int qh = 0; qh < 2; ++qh) {
+            for (int qh = 0; qh < QH; ++qh) {
                 float v = -INFINITY;
 #pragma unroll
                 for (int kt = 0; kt < 2; ++kt)
@@ -765,29 +778,29 @@ __global__ void __launch_bounds__(128 * F5_PAIRS, 1) flash_fwd5_kernel(FaParams 
                     for (int r = 0; r < 16; ++r) v = fmaxf(v, st[kt][qh][r]);
                 vl[qh] = fast_blk ? v : fmaf(v, c_raw, -m_run[qh]);
             }
-            const bool rescale = first || __builtin_amdgcn_ballot_w64(vl[0] > F3_RESCALE || vl[1] > F3_RESCALE) != 0;
-            float sub[2] = {0.f, 0.f};
+            const bool rescale = first || __builtin_amdgcn_ballot_w64(vl[0] > F3_RESCALE || vl[QH - 1] > F3_RESCALE) != 0;
+            float sub[QH] = {};
             if (rescale) {
-                float t[2];
+                float t[QH];
 #pragma unroll
-                for (int qh = 0; qh < 2; ++qh) {
+                for (int qh = 0; qh < QH; ++qh) {
                     float a, bb2;
                     f5_xor32_pair(vl[qh], a, bb2);
                     t[qh] = fmaxf(a, bb2);
                 }
-                float mn[2];
+                float mn[QH];
                 bool ovf = false;
 #pragma unroll
-                for (int qh = 0; qh < 2; ++qh) {
+                for (int qh = 0; qh < QH; ++qh) {
                     // the first block sets m to its maximum (it always holds key 0, so it
                     // is never fully masked); later ones only raise it
                     mn[qh] = m_run[qh] + (first ? t[qh] : fmaxf(t[qh], 0.f));
                     ovf = ovf || !(fabsf(mn[qh]) <= 60000.f);
                 }
                 if (fast && __builtin_amdgcn_ballot_w64(ovf) != 0) fast = false;
-                float alpha[2];
+                float alpha[QH];
 #pragma unroll
-                for (int qh = 0; qh < 2; ++qh) {
+                for (int qh = 0; qh < QH; ++qh) {
                     if (fast) mn[qh] = (float)(f16)mn[qh];
                     alpha[qh] = __builtin_amdgcn_exp2f(m_run[qh] - mn[qh]);
                     sub[qh] = fast_blk ? mn[qh] - m_run[qh] : mn[qh];
@@ -795,12 +808,12 @@ __global__ void __launch_bounds__(128 * F5_PAIRS, 1) flash_fwd5_kernel(FaParams 
                     qm[qh][0] = (fast && h == 0) ? (f16)(-mn[qh]) : (f16)0.f;
                 }
                 if (h == 0) {
-                    abuf[b][pr][r32] = alpha[0];
-                    abuf[b][pr][32 + r32] = alpha[1];
+#pragma unroll
+                    for (int qh = 0; qh < QH; ++qh) abuf[b][pr][32 * qh + r32] = alpha[qh];
                 }
             } else if (!fast_blk) {
-                sub[0] = m_run[0];
-                sub[1] = m_run[1];
+#pragma unroll
+                for (int qh = 0; qh < QH; ++qh) sub[qh] = m_run[qh];
             }
             if (lane == 0) fbuf[b][pr] = rescale ? 1 : 0;
             // P = exp2(S') (or exp2(S c' - m')) in fp16 (RNE), stored as the output wavefront's B operands
@@ -811,7 +824,7 @@ __global__ void __launch_bounds__(128 * F5_PAIRS, 1) flash_fwd5_kernel(FaParams 
 #pragma unroll
                     for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-                        for (int qh = 0; qh < 2; ++qh) {
+                        for (int qh = 0; qh < QH; ++qh) {
                             f5_u32x4 u;
                             const float msub = -sub[qh];
 #pragma unroll
@@ -852,14 +865,14 @@ __global__ void __launch_bounds__(128 * F5_PAIRS, 1) flash_fwd5_kernel(FaParams 
                 vb0[dt] = lds_addr(&vbuf[0][0]) +
                           (uint32_t)((4 * h + jj) * RB + (((4 * dt + 2 * dh + (q >> 1)) ^ (4 * jj)) << 4) + ((q & 1) << 3));
         }
-        f32x16 o[NDT][2];
+        f32x16 o[NDT][QH];
 #pragma unroll
         for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
-            for (int qh = 0; qh < 2; ++qh)
+            for (int qh = 0; qh < QH; ++qh)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) o[dt][qh][r] = 0.f;
-        float l_run[2] = {0.f, 0.f};             // this lane's partial row sums of P
+        float l_run[QH] = {};                    // this lane's partial row sums of P
         const f5_h2 ones = {(_Float16)1.f, (_Float16)1.f};
 
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -872,16 +885,17 @@ __global__ void __launch_bounds__(128 * F5_PAIRS, 1) flash_fwd5_kernel(FaParams 
             dma_tile(false, j + 1);
             if (j <= last) {
                 if (j > 0 && fbuf[b][pr] != 0) {   // the maximum moved at block j: O *= alpha
-                    const float a0 = abuf[b][pr][r32], a1 = abuf[b][pr][32 + r32];
+                    float al[QH];
+#pragma unroll
+                    for (int qh = 0; qh < QH; ++qh) al[qh] = abuf[b][pr][32 * qh + r32];
 #pragma unroll
                     for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
-                        for (int r = 0; r < 16; ++r) {
-                            o[dt][0][r] *= a0;
-                            o[dt][1][r] *= a1;
-                        }
-                    l_run[0] *= a0;
-                    l_run[1] *= a1;
+                        for (int r = 0; r < 16; ++r)
+#pragma unroll
+                            for (int qh = 0; qh < QH; ++qh) o[dt][qh][r] *= al[qh];
+#pragma unroll
+                    for (int qh = 0; qh < QH; ++qh) l_run[qh] *= al[qh];
                 }
                 uint32_t va[NDT];
 #pragma unroll
@@ -902,22 +916,22 @@ __global__ void __launch_bounds__(128 * F5_PAIRS, 1) flash_fwd5_kernel(FaParams 
                 };
                 // V fragments F5_PFV ahead, P one key step ahead; sched_barrier keeps the order
                 f16x8 fr[F5_PFV];
-                f16x8 pp[2][2];   // [kk % 2][qh]
-                pp[0][0] = pread(0, 0);
-                pp[0][1] = pread(0, 1);
+                f16x8 pp[2][QH];   // [kk % 2][qh]
+#pragma unroll
+                for (int qh = 0; qh < QH; ++qh) pp[0][qh] = pread(0, qh);
 #pragma unroll
                 for (int f = 0; f < F5_PFV; ++f) fr[f] = vread(f);
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int i = 0; i < 2 * NVF; ++i) {   // MFMA i: V fragment f = i / 2 (kk = f / NDT, dt = f % NDT), qh = i % 2
-                    const int f = i >> 1, qh = i & 1, kk = f / NDT, dt = f % NDT;
-                    if (i % (2 * NDT) == 0 && kk < 3) {   // the next key step's P fragments
-                        pp[(kk + 1) & 1][0] = pread(kk + 1, 0);
-                        pp[(kk + 1) & 1][1] = pread(kk + 1, 1);
-                    }
-                    if (i % (2 * NDT) == NDT) {   // row sums of this key step's P (fp16 values, fp32 sum)
+                for (int i = 0; i < QH * NVF; ++i) {   // MFMA i: V fragment f = i / QH (kk = f / NDT, dt = f % NDT), qh = i % QH
+                    const int f = i / QH, qh = i % QH, kk = f / NDT, dt = f % NDT;
+                    if (i % (QH * NDT) == 0 && kk < 3) {   // the next key step's P fragments
 #pragma unroll
-                        for (int qq = 0; qq < 2; ++qq)
+                        for (int qq = 0; qq < QH; ++qq) pp[(kk + 1) & 1][qq] = pread(kk + 1, qq);
+                    }
+                    if (i % (QH * NDT) == QH * NDT / 2) {   // row sums of this key step's P (fp16 values, fp32 sum)
+#pragma unroll
+                        for (int qq = 0; qq < QH; ++qq)
 #pragma unroll
                             for (int e = 0; e < 4; ++e)
                                 l_run[qq] = __builtin_amdgcn_fdot2(f5_h2{pp[kk & 1][qq][2 * e], pp[kk & 1][qq][2 * e + 1]},
@@ -925,7 +939,7 @@ __global__ void __launch_bounds__(128 * F5_PAIRS, 1) flash_fwd5_kernel(FaParams 
                     }
                     o[dt][qh] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fr[f % F5_PFV], pp[kk & 1][qh], o[dt][qh], 0, 0,
                                                                        0);
-                    if (qh == 1 && f + F5_PFV < NVF) fr[f % F5_PFV] = vread(f + F5_PFV);
+                    if (qh == QH - 1 && f + F5_PFV < NVF) fr[f % F5_PFV] = vread(f + F5_PFV);
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }
@@ -933,46 +947,45 @@ __global__ void __launch_bounds__(128 * F5_PAIRS, 1) flash_fwd5_kernel(FaParams 
             __syncthreads();
         }
         // ---- O / L, fp16.  o[dt][qh] register r: d = 32 dt + 8 (r / 4) + 4 h + r % 4 of query q0 + 32 qh + r32.
-        float inv[2];
+        float inv[QH];
 #pragma unroll
-        for (int qh = 0; qh < 2; ++qh) {
+        for (int qh = 0; qh < QH; ++qh) {
             float la, lb;
             f5_xor32_pair(l_run[qh], la, lb);
             inv[qh] = 1.f / (la + lb);
         }
         if (p.o16) {
-            // Staged through this pair's P buffers (no wavefront reads them after the last
-            // barrier) as 64 rows of 256 bytes, chunk ^ row % 16, then stored 4 whole rows per
+            // Staged through the Q rows' place (no wavefront reads it after the last barrier) as
+            // rows of 256 bytes, chunk ^ row % 16, then stored 4 whole rows per
             // instruction (16 bytes per lane) instead of 32 rows x 16 bytes.
-            const uint32_t ost[2] = {lds_addr(&pbuf[0][pr][0]), lds_addr(&pbuf[1][pr][0])};
             typedef __attribute__((address_space(3))) f16x4 lds_f16x4;
 #pragma unroll
-            for (int qh = 0; qh < 2; ++qh)
+            for (int qh = 0; qh < QH; ++qh)
 #pragma unroll
                 for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
                     for (int g4 = 0; g4 < 4; ++g4) {
                         const f16x4 v = {(f16)(o[dt][qh][4 * g4 + 0] * inv[qh]), (f16)(o[dt][qh][4 * g4 + 1] * inv[qh]),
                                          (f16)(o[dt][qh][4 * g4 + 2] * inv[qh]), (f16)(o[dt][qh][4 * g4 + 3] * inv[qh])};
-                        *(lds_f16x4*)(uintptr_t)(ost[qh] + (uint32_t)(r32 * RB + (((4 * dt + g4) ^ (r32 & 15)) << 4) + 8 * h)) = v;
+                        *(lds_f16x4*)(uintptr_t)(xst[qh] + (uint32_t)(r32 * RB + (((4 * dt + g4) ^ (r32 & 15)) << 4) + 8 * h)) = v;
                     }
             // all 16 rows of a lane group read before the first store (one LDS round trip), one
             // 64-bit base per lane and a row stride
             const int lrow = lane / CH, cc = lane % CH;
-            f16x8 rv[16];
+            f16x8 rv[8 * QH];
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
+            for (int i = 0; i < 8 * QH; ++i) {
                 const int row = 4 * i + lrow;
-                rv[i] = *(const lds_f16x8*)(uintptr_t)(ost[i / 8] + (uint32_t)((row % 32) * RB + ((cc ^ (row & 15)) << 4)));
+                rv[i] = *(const lds_f16x8*)(uintptr_t)(xst[i / 8] + (uint32_t)((row % 32) * RB + ((cc ^ (row & 15)) << 4)));
             }
             f16* obase = Ob + (int64_t)(q0 + lrow) * p.osl + 8 * cc;
 #pragma unroll
-            for (int i = 0; i < 16; ++i)
+            for (int i = 0; i < 8 * QH; ++i)
                 if (q0 + 4 * i + lrow < p.S && cc < dch)
                     __builtin_nontemporal_store(rv[i], reinterpret_cast<f16x8*>(obase + (int64_t)(4 * i) * p.osl));
         } else {
 #pragma unroll
-            for (int qh = 0; qh < 2; ++qh) {
+            for (int qh = 0; qh < QH; ++qh) {
                 const int q = q0 + 32 * qh + r32;
                 if (q >= p.S) continue;
                 f16* orow = Ob + (int64_t)q * p.osl;
@@ -1020,6 +1033,27 @@ __global__ void flash_generic_kernel(FaParams p, int D) {
     }
     f16* o = p.O + h * p.osh + b * p.osb + (int64_t)qrow * p.osl;
     for (int e = 0; e < D; ++e) o[e] = (f16)(acc[e] / l);
+}
+
+// Whether the score/output kernel runs its 32-query pairs (128 queries a workgroup) instead of the
+// 64-query ones.  A 64-key block costs a workgroup of 32-query pairs about 0.70 (D > 96) or 0.75
+// of what it costs one of 64-query pairs, and a workgroup's start and end about 1.5 such blocks, so
+// twice the workgroups pay where the wide ones leave CUs idle or, causal, the longest of them (its
+// last query block's ceil(S / 64) key blocks) outlasts the rest.  Measured (us, 64- / 32-query pairs;
+// causal but for the last two): B = 1, H = 32, S = 1537, D = 128 37.8 / 29.4; S = 2048 49.3 / 41.3;
+// H = 8, S = 2048 44.0 / 30.1; B = 2, H = 16, S = 512 16.3 / 11.6; but B = 4, H = 32, S = 512 19.2 /
+// 21.4, 1024 54.8 / 58.2, 4096 504 / 598; H = 4, S = 4096, D = 64 64.0 / 48.0; B = 4, H = 12, S = 777,
+// D = 64 18.1 / 25.9.
+static bool fa_narrow_preferred(int64_t S, int64_t heads, int64_t D, bool causal) {
+    auto cost = [&](int64_t bq, double block) {
+        const double nqb = (double)((S + bq - 1) / bq), nkb = (double)((S + F5_BK - 1) / F5_BK);
+        const double wgs = nqb * (double)heads, per = (double)(bq / F5_BK), rounds = std::ceil(wgs / 256);
+        // key blocks on the busiest CU: causal, a head's sum spread over the CUs, or its longest one
+        const double sum = per * nqb * (nqb + 1) / 2 - (nqb * per - nkb);
+        const double blocks = causal ? std::max(nkb, sum * (double)heads / 256) : rounds * nkb;
+        return block * blocks + 1.5 * rounds;
+    };
+    return cost(32 * F5_PAIRS, D > 96 ? 0.70 : 0.75) < cost(64 * F5_PAIRS, 1.0);
 }
 
 }  // namespace lava
@@ -1081,7 +1115,7 @@ extern "C" int lava_hip_flash_attn_fwd_f16(const void* Q, const void* K, const v
     lay_ok = lay_ok && aligned(Q, 16) && aligned(K, 16) && aligned(V, 16) && aligned(O, 8) &&
              S * strides[1] * 2 < ((int64_t)1 << 31);
     const int64_t blocks3 = ((S + F3_BQ - 1) / F3_BQ) * H * B;
-    const int64_t blocks5 = ((S + F5_BQ - 1) / F5_BQ) * H * B;
+    const int64_t blocks5 = ((S + 32 * F5_PAIRS - 1) / (32 * F5_PAIRS)) * H * B;   // with 32-query pairs, the most
     const int pin = kernel_override(LAVA_HIP_FAMILY_ATTN);
     const bool fast3 = lay_ok && scale > 0.f && (D == 64 || D == FA_D) && pin == 3 && blocks3 <= 0x7fffffff;
     const bool fast5 = lay_ok && !fast3 && blocks5 <= 0x7fffffff;
@@ -1093,16 +1127,24 @@ extern "C" int lava_hip_flash_attn_fwd_f16(const void* Q, const void* K, const v
                    S * strides[1] * 2 < ((int64_t)1 << 31);
     for (int i = 1; i < 4; ++i) fast256 = fast256 && strides[i] % 8 == 0 && os[i] % 4 == 0;
     if (fast5) {   // any D <= 128, a multiple of 8 (staged zero-padded to 128; MFMAs over D rounded up to 64, 96, 128)
-        auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3((unsigned)blocks5), dim3(128 * F5_PAIRS), 0, s, p); };
-        if (p.causal) {
-            if (D <= 64) go(flash_fwd5_kernel<true, 64>);
-            else if (D <= 96) go(flash_fwd5_kernel<true, 96>);
-            else go(flash_fwd5_kernel<true, 128>);
-        } else {
-            if (D <= 64) go(flash_fwd5_kernel<false, 64>);
-            else if (D <= 96) go(flash_fwd5_kernel<false, 96>);
-            else go(flash_fwd5_kernel<false, 128>);
-        }
+        auto go = [&](auto kernel, int64_t blocks) {
+            hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(128 * F5_PAIRS), 0, s, p);
+        };
+        auto by_d = [&](auto causal_tag, auto qh_tag) {
+            constexpr bool C = decltype(causal_tag)::value;
+            constexpr int QH = decltype(qh_tag)::value;
+            const int64_t blocks = ((S + 32 * QH * F5_PAIRS - 1) / (32 * QH * F5_PAIRS)) * H * B;
+            if (D <= 64) go(flash_fwd5_kernel<C, 64, QH>, blocks);
+            else if (D <= 96) go(flash_fwd5_kernel<C, 96, QH>, blocks);
+            else go(flash_fwd5_kernel<C, 128, QH>, blocks);
+        };
+        const bool narrow = fa_narrow_preferred(S, H * B, D, p.causal);
+        typedef std::integral_constant<int, 1> Q1;
+        typedef std::integral_constant<int, 2> Q2;
+        if (p.causal)
+            narrow ? by_d(f3_tag<true>{}, Q1{}) : by_d(f3_tag<true>{}, Q2{});
+        else
+            narrow ? by_d(f3_tag<false>{}, Q1{}) : by_d(f3_tag<false>{}, Q2{});
         LAVA_LAUNCH_CHECK("flash_fwd5_kernel");
         return LAVA_HIP_OK;
     }

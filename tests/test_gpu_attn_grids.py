@@ -1,0 +1,39 @@
+"""Both widths of the score/output attention kernel: grids that give its 64-query pairs (many heads)
+and its 32-query ones (few), with S at the edges of a key block, a 128- and a 256-query workgroup.
+Reference: softmax in 64 bits; bar: the attention configurations' relative Frobenius error of 2e-3
+(fp16 probabilities and result, 2^-11 each)."""
+import math
+
+import numpy as np
+import pytest
+
+from conftest import announce
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("H,B", [(32, 16), (3, 1)])
+@pytest.mark.parametrize("E", [32, 64, 80, 128])
+@pytest.mark.parametrize("L", [1, 33, 64, 97, 129, 192, 256, 321])
+def test_flash_both_widths(gpu, E, L, H, B, causal):
+    lh = gpu
+    announce(f"flash widths D={E} S={L} H={H} B={B} causal={causal}")
+    rng = np.random.default_rng(E + L + H)
+    q, k, v = (np.asfortranarray(rng.standard_normal((E, L, H, B)).astype(np.float16)) for _ in range(3))
+    Q, K, V = (lh.HIPDeviceArray.from_numpy(t, "f16") for t in (q, k, v))
+    O = lh.HIPDeviceArray("f16", (E, L, H, B))
+    O.fill_bytes(0xFF)
+    lh.kernel_log_clear()
+    lh.flash_attn_fwd(O, Q, K, V, causal=causal)
+    assert "flash_fwd5_kernel" in lh.kernel_log() or E == 64, lh.kernel_log()
+    got = O.to_numpy()
+    assert not np.isnan(got).any()
+    for h, b in {(0, 0), (H - 1, B - 1), (H // 2, B // 2)}:
+        s = q[:, :, h, b].T.astype(np.float64) @ k[:, :, h, b].astype(np.float64) / math.sqrt(E)
+        if causal:
+            s = np.where(np.tril(np.ones((L, L), bool)), s, -np.inf)
+        p = np.exp(s - s.max(axis=1, keepdims=True))
+        want = (p / p.sum(axis=1, keepdims=True)) @ v[:, :, h, b].T.astype(np.float64)
+        err = np.linalg.norm(got[:, :, h, b].T - want) / np.linalg.norm(want)
+        assert err <= 2e-3, (h, b, err)
