@@ -86,6 +86,12 @@ int mid_gemm_eligible(const void* A, const void* B, const void* C, int64_t M, in
 template <typename T, typename OutT, bool EPI, bool U8 = false>
 int launch_gemm_mid(const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
                     int64_t ldc, hipStream_t s, const Epilogue& epi, bool ragged, bool ak, bool bk);
+// The mid-size kernel's K-split form (gemm_mid_ksplit.hip): plain products, the operands and extents
+// of mid_gemm_eligible; and whether an eligible product runs on it (it then leads all the others).
+template <typename T>
+int launch_gemm_mid_ksplit(const T* A, const T* B, typename Mfma16<T>::acc_elem* C, int64_t M, int64_t N, int64_t K,
+                           int64_t lda, int64_t ldb, int64_t ldc, hipStream_t s, bool ragged, bool ak, bool bk);
+bool mid_ksplit_preferred(int64_t M, int64_t N, int64_t k_bytes);
 // Whether an M x N product takes the mid-size kernel when it fits (the measured choice against the
 // tile and small-product kernels).
 bool mid_gemm_preferred(int64_t M, int64_t N);

@@ -192,7 +192,7 @@ struct TnSide<T, false, 128> {
     int klim;          // instruction i's row is inside iff k0 + 4 i < klim
     bool cin[2];       // the lane's chunk lies inside M (N), per variant
     int mr16;          // fragment reads: the lane's row and byte offset
-    int c16[4];        // fragment reads: the stored chunk of column block t, times 16
+    int c16[4];        // fragment reads: the stored chunk of column block t, times 16 (t above 3: see read16)
 
     __device__ __forceinline__ static int swz(int r) { return 2 * (r & 3) + 8 * (((r >> 3) ^ (r >> 4)) & 1); }
 
@@ -321,7 +321,7 @@ struct TnSide<int8_t, false, 128> {
     int klim;          // instruction i's row is inside iff k0 + 8 i < klim
     bool cin[2];       // the lane's chunk lies inside M (N), per variant
     int rd;            // fragment reads: the lane's k row and byte offset
-    int c16[4];        // fragment reads: the stored chunk of column block t, times 16
+    int c16[4];        // fragment reads: the stored chunk of column block t, times 16 (t above 3: see read16)
 
     __device__ __forceinline__ static int swz(int r) { return ((r >> 1) & 3) | ((((r >> 4) ^ (r >> 5)) & 1) << 2); }
 
@@ -357,7 +357,8 @@ struct TnSide<int8_t, false, 128> {
     // fragment t (columns 16 t of the half) of k-step u (64 rows of K): two transposing reads,
     // k rows 16 g + [0, 8) and 16 g + [8, 16) of the k-step
     __device__ __forceinline__ uint4 read16(const uint8_t* slice, int u, int t) const {
-        const uint8_t* b = slice + u * 64 * 128 + rd + c16[t];
+        // (blocks 4 to 7 are the other half's: their chunks differ in the slot's top bit)
+        const uint8_t* b = slice + u * 64 * 128 + rd + (t < 4 ? c16[t & 3] : c16[t & 3] ^ 64);
         const tn_v2i lo = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
             (__attribute__((address_space(3))) tn_v2i*)(const __attribute__((address_space(3))) uint8_t*)b);
         const tn_v2i hi = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
