@@ -8,7 +8,9 @@
 // zero-clamped loads.  Mid-size products, plain or with the fused epilogue (at least 128 tiles of
 // 128 x 128 and fewer than 144 of 256 x 256, or 257 to 336 of them: mid_gemm_preferred), take the
 // 128 x 128 kernel (gemm_mid_kernel.hpp), at most 256 tiles with a long K (and some of 65 to 127 tiles,
-// mid_ksplit_preferred) in its K-split form (gemm_mid_ksplit.hip).  Other products of at most 16
+// mid_ksplit_preferred) in its K-split form (gemm_mid_ksplit.hip).  Products of at most 64 rows or
+// columns whose 64 x 64 tiles fill the CUs about once, or whose K is too short to split, take
+// gemm_skinny.hip (skinny_gemm_preferred).  Other products of at most 16
 // tiles of 256 x 256, and products that the tile kernel would run on few CUs or mostly empty
 // tiles (small_gemm_preferred's rate estimate), take the 64 x 64 small-product kernel (with K
 // split over the stream's workspace where its tiles alone would leave CUs idle:
@@ -81,6 +83,10 @@ int gemm_entry(const char* name, const void* A, const void* B, void* C, int64_t 
     // the 128 x 128 mid-size kernel: plain output, the fused epilogue (f16 / bf16) or unsigned bytes
     if constexpr (EPI || std::is_same<OutT, typename Mfma16<T>::acc_elem>::value) {
         const int mfit = mid_gemm_eligible<T>(a, b, c, M, N, K, lda, ldb, ldc, sizeof(OutT), arow, !brow);
+        if constexpr (!EPI && !U8) {
+            if (mfit != TN_NO && pin == 0 && skinny_gemm_preferred(M, N, K * (int64_t)sizeof(T), sizeof(T), arow, !brow))
+                return launch_gemm_skinny<T>(a, b, c, M, N, K, lda, ldb, ldc, s, arow, !brow);
+        }
         const bool ksplit = !EPI && !U8 && mid_ksplit_preferred(M, N, K * (int64_t)sizeof(T));
         if (mfit != TN_NO && (pin == 4 || (pin == 0 && (ksplit || mid_gemm_preferred(M, N))))) {
             if constexpr (!EPI && !U8) {
