@@ -151,10 +151,10 @@ __device__ __forceinline__ uint4 any_shift(uint4 x, int bits) {
 // height has no two rows aligned alike).  A thread's 16 bytes are then one load of element
 // alignment, always whole and always inside the matrix: a chunk that would pass the end of its row
 // (K, M or N) is read from the row's last 16 bytes instead, a row past the last from the last row,
-// both from clamped addresses, so every load of a K chunk is in flight at once without a branch.  On
-// the way into LDS the pulled-back chunks are shifted down into place with zeros behind the end of
+// both from clamped addresses; a chunk wholly past K is not read (a short last K chunk then costs
+// what it holds: 19.1 -> 17.1 us below).  On the way into LDS the pulled-back chunks are shifted down into place with zeros behind the end of
 // K (any_shift), only in workgroups and K chunks that reach an end.  Bound by the latency of a chunk's
-// loads, like the aligned form; fp16, all column-major, 1111 x 1333 x 777: 18.5 us a call (125
+// loads, like the aligned form; fp16, all column-major, 1111 x 1333 x 777: 17.1 us a call (134
 // TFLOP/s) against 99.3 on the staged kernel, which loads element by element.
 template <typename T, bool AROW, bool BROW, typename OutT, bool EPI, bool U8 = false, bool ANY = false>
 __global__ void __launch_bounds__(256) gemm_small_kernel(const T* __restrict__ A, const T* __restrict__ B,
@@ -195,16 +195,21 @@ __global__ void __launch_bounds__(256) gemm_small_kernel(const T* __restrict__ A
             int64_t rr, kk;
             const T* p;
             if constexpr (ANY) {
+                bool in;   // chunks wholly past K stay zero
                 if constexpr (decltype(kcont)::value) {
+                    const int64_t k1 = k0 + (int64_t)EV * (e & 31);
+                    in = k1 < ke;
                     rr = min(r0 + (e >> 5), rows - 1);
-                    kk = min(k0 + (int64_t)EV * (e & 31), ke - EV);
+                    kk = min(k1, ke - EV);
                     p = X + rr * ld + kk;
                 } else {
-                    kk = min(k0 + e / JR, ke - 1);
+                    kk = k0 + e / JR;
+                    in = kk < ke;
                     rr = min(r0 + (int64_t)EV * (e % JR), rows - EV);
                     p = X + kk * ld + rr;
                 }
-                reg[i] = any_load(p);
+                reg[i] = make_uint4(0, 0, 0, 0);
+                if (in) reg[i] = any_load(p);
                 continue;
             }
             if constexpr (decltype(kcont)::value) {
@@ -235,7 +240,6 @@ __global__ void __launch_bounds__(256) gemm_small_kernel(const T* __restrict__ A
             uint4 x = reg[i];
             if constexpr (ANY) {
                 if (decltype(kcont)::value ? k_end : r_end) x = any_shift(x, shift * 8 * (int)sizeof(T));
-                if (!decltype(kcont)::value && k_end && k0 + e / JR >= ke) x = make_uint4(0, 0, 0, 0);
             }
             if constexpr (U8) {
                 x.x ^= 0x80808080u;
@@ -490,8 +494,8 @@ bool small_gemm_fits(const void* A, const void* B, int64_t M, int64_t N, int64_t
            ((arow || !brow) ? K % EV == 0 : true) && (arow || M % EV == 0) && (!brow || N % EV == 0);
 }
 // The ANY form reads 16 bytes inside each row, so the contiguous extent of each operand holds at
-// least that much; nothing else is asked of it.  It leads the staged kernel wherever it fits (99.3 ->
-// 18.5 us at 1111 x 1333 x 777); the aligned forms lead it, so it runs where none of them fits.
+// least that much; nothing else is asked of it.  It leads the staged kernel wherever it fits (99.4 ->
+// 17.1 us at 1111 x 1333 x 777); the aligned forms lead it, so it runs where none of them fits.
 template <typename T>
 bool small_any_fits(int64_t M, int64_t N, int64_t K, bool arow, bool brow) {
     constexpr int64_t EV = 16 / (int64_t)sizeof(T);
