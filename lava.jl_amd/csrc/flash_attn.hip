@@ -10,6 +10,8 @@
 // Kernels (the dispatcher at the end of the file picks one):
 //  * flash_fwd5_kernel -- D <= 128 (the headline shape D = 128), any softmax scale: on each SIMD
 //    a score wavefront and an output wavefront share 64 queries (described at the kernel);
+//  * flash_fwd6_kernel -- D = 56 and 64 with a positive scale, where it is the faster one (fa_cost):
+//    64 queries' both products in each wavefront, two wavefronts splitting the key blocks;
 //  * flash_fwd3_kernel -- D = 256 with a positive scale (and D = 64 or 128 on request):
 //    ping-pong pairs of 32-query wavefronts;
 //  * flash_generic_kernel -- any D <= 256, one thread per query (every other case).
@@ -516,7 +518,7 @@ __global__ void __launch_bounds__(64 * F3_WAVES, 1) flash_fwd3_kernel(FaParams p
 // the softmax.
 // QH = 1 gives each pair one 32-query half (128 queries per workgroup): a fragment then feeds one MFMA
 // and a key block takes 0.70 of the time for half the queries, for grids that 256-query workgroups
-// leave uneven or short of the 256 CUs (fa_narrow_preferred).
+// leave uneven or short of the 256 CUs (fa_cost).
 constexpr int F5_PAIRS = 4;
 constexpr int F5_BK = 64;
 constexpr int F5_KST = 3, F5_VST = 2;
@@ -1003,6 +1005,348 @@ __global__ void __launch_bounds__(128 * F5_PAIRS, 1) flash_fwd5_kernel(FaParams 
     }
 }
 
+// ---- flash_fwd6_kernel: head dimensions 56 and 64, both products in one wavefront ----
+//
+// At D = 64 a 64-key block has half the MFMAs of D = 128 and the same softmax.  O^T (64 registers), the
+// scores (64), Q^T (32) and -m (32) of 64 queries fit one wavefront at two per SIMD, so each wavefront
+// does both products and the softmax and P stays in registers (the score accumulator converts in
+// place to the second product's operand) instead of crossing LDS between a score and an output
+// wavefront:
+//  * 8 wavefronts: 4 groups of 32 QH queries, each by two wavefronts (w and w + 4, one SIMD) that take
+//    the even and the odd key blocks and merge their sums at the end through LDS, so a workgroup's
+//    chain is half its key blocks;
+//  * a step is two key blocks: K and V of both, 32 KB (128-byte rows, not padded to 256), by LDS-DMA
+//    in a ring of four; one barrier a step, a request has two steps to land;
+//  * -m is the score product's initial accumulator, so P = exp2 of the scores as they come (the base-2
+//    scale is folded into Q^T); each 16-key step's exponentials sit between the second product's MFMAs
+//    of the step before;
+//  * lazy rescaling as in the other kernels.
+// What bounds it is issue: 208 VALU instructions and 32 MFMAs per 64-query block take about 2250 cycles
+// of a SIMD (MFMA busy 0.43), and taking out the exponentials, the maximum or the row sums (timing
+// copies) gained 4, 3 and 3 %; half a step's offset between a SIMD's wavefronts, four 32-query
+// wavefronts a SIMD, and the scale and maximum as a multiply-add per score all ran within 5 % of it.
+// B = 4, H = 32, S = 4096 343 -> 323 us causal, 625 -> 573 not; with 32-query groups (QH = 1) H = 4, S =
+// 4096 not causal 47.7 -> 37.6, B = 2, H = 12, S = 1500 causal 22.6 -> 18.3 (fa_cost has the rule).
+// D = 56 runs zero-padded to 64 (chunks past D read zero).
+constexpr int F6_GROUPS = 4;
+constexpr int F6_TILE = F5_BK * 128;        // 64 keys of 128 bytes
+constexpr int F6_STEP = 4 * F6_TILE;        // K, K, V, V of two blocks
+constexpr int F6_RING = 4;
+
+template <bool CAUSAL, int QH>
+__global__ void __launch_bounds__(512, 1) flash_fwd6_kernel(FaParams p) {
+    constexpr int RB = 128, PQ = 32 * QH, BQ = PQ * F6_GROUPS;
+    __shared__ __attribute__((aligned(1024))) uint8_t ring[F6_RING][F6_STEP];
+    __shared__ float2 stat[8][QH][32];
+
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int gq = w & 3, kh = w >> 2;         // query group, key half
+    const int r32 = lane & 31, h = lane >> 5;
+    const int nqb = (p.S + BQ - 1) / BQ;
+    int bh, qb;
+    fa_order(nqb, p.H * p.B, CAUSAL, bh, qb);
+    const int hh = bh % p.H, bb = bh / p.H;
+    const int64_t head = (int64_t)hh * p.sh + (int64_t)bb * p.sb;
+    f16* Ob = p.O + (int64_t)hh * p.osh + (int64_t)bb * p.osb;
+    const int q0 = qb * BQ + gq * PQ;
+    const int nkb_s = (p.S + F5_BK - 1) / F5_BK;
+    const int nkb = CAUSAL ? min((qb * BQ + BQ - 1) / F5_BK + 1, nkb_s) : nkb_s;
+    const int last = CAUSAL ? min(nkb - 1, (q0 + PQ - 1) / F5_BK) : nkb - 1;   // this group's last key block
+    const int steps = (nkb + 1) / 2;
+
+    // LDS-DMA: wavefront w moves rows 8 w + lane / 8 of each of a step's four tiles, slot lane % 8
+    // (K chunk ^ row % 8 ^ row / 8 % 2, V chunk ^ 2 (row % 4)); rows at or past S and chunks at or past
+    // D read zero
+    const uint32_t row_bytes = (uint32_t)(p.sl * 2);
+    const int dch = p.D >> 3;
+    const int lr = lane >> 3, slot = lane & 7;
+    auto chunk_ofs = [&](int row, int c) -> uint32_t {
+        return c < dch ? (uint32_t)row * row_bytes + 16u * (uint32_t)c : 0x80000000u;
+    };
+    const uint32_t ofs_k = chunk_ofs(8 * w + lr, slot ^ lr ^ (w & 1)), ofs_v = chunk_ofs(8 * w + lr, slot ^ (2 * (lr & 3)));
+    const uint32_t lds_w = lds_addr(&ring[0][0]) + 1024u * w;
+    auto dma_step = [&](int j, int st) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const int kb = 2 * j + (t & 1);
+            const int first = min(kb, nkb - 1) * F5_BK;
+            const uint32_t rows = kb < nkb ? (uint32_t)min(F5_BK, p.S - first) : 0u;
+            const v4i rs = make_rsrc((t < 2 ? p.K : p.V) + head + (int64_t)first * p.sl, rows * row_bytes);
+            dma16(rs, t < 2 ? ofs_k : ofs_v, 0u, __builtin_amdgcn_readfirstlane(lds_w + (uint32_t)(st * F6_STEP + t * F6_TILE)));
+        }
+    };
+    typedef __attribute__((address_space(3))) f16x8 lds_f16x8;
+    typedef __attribute__((address_space(3))) f3_s16x4 lds_s16x4;
+    typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
+
+    // Q of the group: PQ rows, half by each of its wavefronts, in the K tile's layout, through the
+    // ring's last place (free until the first step)
+    const uint32_t lds_q = lds_addr(&ring[F6_RING - 1][0]) + (uint32_t)(gq * PQ * RB);
+    {
+        const uint32_t rows = (uint32_t)max(0, min(PQ, p.S - q0));
+        const v4i rs = make_rsrc(p.Q + head + (int64_t)q0 * p.sl, rows * row_bytes);
+#pragma unroll
+        for (int i = 0; i < PQ / 16; ++i) {
+            const int i8 = kh * (PQ / 16) + i;   // 8 rows per instruction
+            dma16(rs, chunk_ofs(8 * i8 + lr, slot ^ lr ^ (i8 & 1)), 0u,
+                  __builtin_amdgcn_readfirstlane(lds_q + 1024u * i8));
+        }
+    }
+    dma_step(0, 0);
+    dma_step(1, 1);
+    asm volatile("s_waitcnt vmcnt(4)" ::: "memory");   // Q and step 0
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+
+    // (the first request into Q's place is step 3's, after the first step's barrier)
+    const int ksw = (r32 & 7) ^ ((r32 >> 3) & 1);
+    f16x8 qf[QH][4];   // Q^T B operands: query q0 + 32 qh + r32, d = 16 ks + 8 h + [0, 8)
+#pragma unroll
+    for (int qh = 0; qh < QH; ++qh)
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks)
+            qf[qh][ks] = *(const lds_f16x8*)(uintptr_t)(lds_q + (uint32_t)((32 * qh + r32) * RB + (((2 * ks + h) ^ ksw) << 4)));
+    uint32_t k_rd[4], v_rd[2];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) k_rd[ks] = lds_addr(&ring[0][0]) + (uint32_t)(kh * F6_TILE + r32 * RB + (((2 * ks + h) ^ ksw) << 4));
+    {
+        const int jj = (lane & 15) >> 2, q = lane & 3, dh = (lane >> 4) & 1;
+#pragma unroll
+        for (int dt = 0; dt < 2; ++dt)
+            v_rd[dt] = lds_addr(&ring[0][0]) + (uint32_t)((2 + kh) * F6_TILE + (4 * h + jj) * RB +
+                                                          (((4 * dt + 2 * dh + (q >> 1)) ^ (2 * jj)) << 4) + ((q & 1) << 3));
+    }
+    f32x16 o[2][QH];
+#pragma unroll
+    for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+        for (int qh = 0; qh < QH; ++qh)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o[dt][qh][r] = 0.f;
+    float m_run[QH], l_run[QH];
+#pragma unroll
+    for (int qh = 0; qh < QH; ++qh) {
+        m_run[qh] = 0.f;
+        l_run[qh] = 0.f;
+    }
+    const f5_h2 ones = {(_Float16)1.f, (_Float16)1.f};
+    f32x16 neg_m[QH];   // -m of the lane's query: the score product's initial accumulator
+#pragma unroll
+    for (int qh = 0; qh < QH; ++qh)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) neg_m[qh][r] = 0.f;
+    // the base-2 scale folded into Q^T (c <= 1, so the product cannot overflow; one rounding of q c)
+#pragma unroll
+    for (int qh = 0; qh < QH; ++qh)
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) fa_scale_f16(qf[qh][ks], p.scale_log2);
+
+    auto block = [&](int kb, uint32_t st_ofs, bool first) __attribute__((always_inline)) {
+        f32x16 st[2][QH];   // S' = c q.k - m; st[kt][qh] register r: key 32 kt + 8 (r / 4) + 4 h + r % 4
+        auto kread = [&](int f) __attribute__((always_inline)) -> f16x8 {   // f = 2 ks + kt
+            return *(const lds_f16x8*)(uintptr_t)(k_rd[f >> 1] + st_ofs + (uint32_t)((f & 1) * 32 * RB));
+        };
+        f16x8 fr[4];
+#pragma unroll
+        for (int f = 0; f < 4; ++f) fr[f] = kread(f);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 8 * QH; ++i) {   // fragment f = i / QH, qh = i % QH
+            const int f = i / QH, qh = i % QH, ks = f >> 1, kt = f & 1;
+            st[kt][qh] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fr[f & 3], qf[qh][ks], ks == 0 ? neg_m[qh] : st[kt][qh], 0, 0, 0);
+            if (qh == QH - 1 && f + 4 < 8) fr[f & 3] = kread(f + 4);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        auto vread = [&](int f) __attribute__((always_inline)) -> f16x8 {   // f = 2 kk + dt, keys 16 kk ..
+            const int kk = 16 * (f >> 1), dt = f & 1;
+            const f3_s16x4 lo =
+                __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(uintptr_t)(v_rd[dt] + st_ofs + (uint32_t)(kk * RB)));
+            const f3_s16x4 hi =
+                __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(uintptr_t)(v_rd[dt] + st_ofs + (uint32_t)((kk + 8) * RB)));
+            return __builtin_bit_cast(f16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        };
+        f16x8 vf[4];
+#pragma unroll
+        for (int f = 0; f < 4; ++f) vf[f] = vread(f);
+        // mask: causal key > query (the group's last block holds its diagonal); else keys >= S
+        if (CAUSAL ? kb == last : (kb + 1) * F5_BK > p.S) {
+            int dv = CAUSAL ? kb * F5_BK + 4 * h - r32 - q0 : kb * F5_BK + 4 * h - p.S;
+            asm volatile("; mask" : "+v"(dv));
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+                for (int qh = 0; qh < QH; ++qh)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const int kr = 32 * kt + 8 * (r >> 2) + (r & 3);
+                        const bool off = CAUSAL ? dv > 32 * qh - kr : dv >= -kr;
+                        st[kt][qh][r] = off ? -INFINITY : st[kt][qh][r];
+                    }
+        }
+        float vl[QH];   // this lane's largest S' per query half
+        bool up = first;
+#pragma unroll
+        for (int qh = 0; qh < QH; ++qh) {
+            float v = -INFINITY;
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) v = fmaxf(v, st[kt][qh][r]);
+            vl[qh] = v;
+            up = up || v > F3_RESCALE;
+        }
+        if (__builtin_amdgcn_ballot_w64(up) != 0) {
+#pragma unroll
+            for (int qh = 0; qh < QH; ++qh) {
+                float a, b;
+                f5_xor32_pair(vl[qh], a, b);
+                // the first block sets m to its maximum (finite: a block's first key is never masked),
+                // later ones only raise it
+                const float t = fmaxf(a, b), d = first ? t : fmaxf(t, 0.f);
+                const float alpha = first ? 1.f : __builtin_amdgcn_exp2f(-d);
+                m_run[qh] += d;
+                l_run[qh] *= alpha;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    neg_m[qh][r] = -m_run[qh];
+                    st[0][qh][r] -= d;
+                    st[1][qh][r] -= d;
+                    o[0][qh][r] *= alpha;
+                    o[1][qh][r] *= alpha;
+                }
+            }
+        }
+        // P of key step kk (16 keys) and its row sums
+        f5_u32x4 pf[2][QH];
+        auto probs = [&](int kk, int qh) __attribute__((always_inline)) {
+            f5_u32x4 u;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int r0 = 8 * (kk & 1) + 2 * k;
+                const f5_h2 hv = {(_Float16)__builtin_amdgcn_exp2f(st[kk >> 1][qh][r0]),
+                                  (_Float16)__builtin_amdgcn_exp2f(st[kk >> 1][qh][r0 + 1])};
+                l_run[qh] = __builtin_amdgcn_fdot2(hv, ones, l_run[qh], false);
+                u[k] = __builtin_bit_cast(uint32_t, hv);
+            }
+            pf[kk & 1][qh] = u;
+        };
+#pragma unroll
+        for (int qh = 0; qh < QH; ++qh) probs(0, qh);
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) {
+#pragma unroll
+            for (int qh = 0; qh < QH; ++qh) {
+#pragma unroll
+                for (int dt = 0; dt < 2; ++dt)
+                    o[dt][qh] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                        vf[(2 * kk + dt) & 3], __builtin_bit_cast(f16x8, pf[kk & 1][qh]), o[dt][qh], 0, 0, 0);
+                if (kk < 3) probs(kk + 1, qh);
+            }
+            if (kk < 2) {
+                vf[(2 * kk) & 3] = vread(2 * kk + 4);
+                vf[(2 * kk + 1) & 3] = vread(2 * kk + 5);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+
+    for (int j = 0; j < steps; ++j) {
+        const uint32_t now = (uint32_t)((j & (F6_RING - 1)) * F6_STEP);
+        dma_step(j + 2, (j + 2) & (F6_RING - 1));
+        const int kb = 2 * j + kh;
+        if (kb <= last) block(kb, now, j == 0);
+        asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");   // this wavefront's part of step j + 1 landed
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+
+    // ---- merge.  Of its two partial results a group's wavefront kh finishes query half kh (QH = 2) or
+    // columns 32 kh .. + 31 (QH = 1) and hands over the rest; a wavefront with no block has m = -inf
+    // and weighs nothing.
+    constexpr int ND = QH == 2 ? 2 : 1;   // 32-column tiles this wavefront finishes
+    f32x16 keep[ND];
+    const int peer = w ^ 4;
+    auto box = [&](int wave) { return lds_addr(&ring[0][0]) + (uint32_t)(wave * ND * 4096 + lane * 16); };
+#pragma unroll
+    for (int t = 0; t < ND; ++t) {
+        f32x16 give;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const float lo = QH == 2 ? o[t][0][r] : o[0][0][r], hi = QH == 2 ? o[t][QH - 1][r] : o[1][0][r];
+            keep[t][r] = kh ? hi : lo;
+            give[r] = kh ? lo : hi;
+        }
+#pragma unroll
+        for (int g4 = 0; g4 < 4; ++g4)
+            *(lds_f32x4*)(uintptr_t)(box(w) + (uint32_t)(t * 4 + g4) * 1024u) =
+                f32x4{give[4 * g4], give[4 * g4 + 1], give[4 * g4 + 2], give[4 * g4 + 3]};
+    }
+    float l_all[QH];
+#pragma unroll
+    for (int qh = 0; qh < QH; ++qh) {
+        float a, b;
+        f5_xor32_pair(l_run[qh], a, b);
+        l_all[qh] = a + b;
+        if (h == 0) stat[w][qh][r32] = make_float2(kh <= last ? m_run[qh] : -INFINITY, l_all[qh]);
+    }
+    __syncthreads();
+    const int mq = QH == 2 ? kh : 0;
+    const float m_own = kh > last ? -INFINITY : (QH == 2 && kh ? m_run[QH - 1] : m_run[0]), l_own = QH == 2 && kh ? l_all[QH - 1] : l_all[0];
+    const float2 ot = stat[peer][mq][r32];
+    const float m_all = fmaxf(m_own, ot.x);
+    const float a_own = __builtin_amdgcn_exp2f(m_own - m_all), a_ot = __builtin_amdgcn_exp2f(ot.x - m_all);
+    const float inv = 1.f / (a_own * l_own + a_ot * ot.y);
+    const float f_own = a_own * inv, f_ot = a_ot * inv;
+#pragma unroll
+    for (int t = 0; t < ND; ++t)
+#pragma unroll
+        for (int g4 = 0; g4 < 4; ++g4) {
+            const f32x4 x = *(const lds_f32x4*)(uintptr_t)(box(peer) + (uint32_t)(t * 4 + g4) * 1024u);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) keep[t][4 * g4 + r] = keep[t][4 * g4 + r] * f_own + x[r] * f_ot;
+        }
+    const int qs = q0 + (QH == 2 ? 32 * kh : 0), c0 = QH == 2 ? 0 : 4 * kh;   // first query, first 16-byte chunk
+    if (p.o16) {
+        // rows of 16 ND x 4 bytes staged behind the boxes, chunk ^ row % (4 ND), then stored whole
+        constexpr int NC = 4 * ND;
+        const uint32_t ep = lds_addr(&ring[0][0]) + (uint32_t)(8 * ND * 4096 + w * 32 * NC * 16);
+        typedef __attribute__((address_space(3))) f16x4 lds_f16x4;
+#pragma unroll
+        for (int t = 0; t < ND; ++t)
+#pragma unroll
+            for (int g4 = 0; g4 < 4; ++g4) {
+                const f16x4 v = {(f16)keep[t][4 * g4], (f16)keep[t][4 * g4 + 1], (f16)keep[t][4 * g4 + 2], (f16)keep[t][4 * g4 + 3]};
+                *(lds_f16x4*)(uintptr_t)(ep + (uint32_t)((r32 * NC + ((4 * t + g4) ^ (r32 & (NC - 1)))) * 16 + 8 * h)) = v;
+            }
+        __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
+        __builtin_amdgcn_wave_barrier();
+        constexpr int RPI = 64 / NC;
+        const int row = lane / NC, cc = lane % NC;
+        f16x8 rv[32 / RPI];
+#pragma unroll
+        for (int i = 0; i < 32 / RPI; ++i)
+            rv[i] = *(const lds_f16x8*)(uintptr_t)(ep + (uint32_t)(((RPI * i + row) * NC + (cc ^ ((RPI * i + row) & (NC - 1)))) * 16));
+        f16* obase = Ob + (int64_t)(qs + row) * p.osl + 8 * (c0 + cc);
+#pragma unroll
+        for (int i = 0; i < 32 / RPI; ++i)
+            if (qs + RPI * i + row < p.S && c0 + cc < dch)
+                __builtin_nontemporal_store(rv[i], reinterpret_cast<f16x8*>(obase + (int64_t)(RPI * i) * p.osl));
+    } else if (qs + r32 < p.S) {
+        f16* orow = Ob + (int64_t)(qs + r32) * p.osl;
+#pragma unroll
+        for (int t = 0; t < ND; ++t)
+#pragma unroll
+            for (int g4 = 0; g4 < 4; ++g4) {
+                const int d = 8 * (c0 + 4 * t + g4) + 4 * h;
+                const f16x4 v = {(f16)keep[t][4 * g4], (f16)keep[t][4 * g4 + 1], (f16)keep[t][4 * g4 + 2], (f16)keep[t][4 * g4 + 3]};
+                if (d < p.D) __builtin_nontemporal_store(v, reinterpret_cast<f16x4*>(orow + d));
+            }
+    }
+}
+
 // Any D <= 256, any S: one thread per query row, online softmax in fp32 over every
 // key (the clamped/ragged path; not the fast one).
 __global__ void flash_generic_kernel(FaParams p, int D) {
@@ -1035,8 +1379,8 @@ __global__ void flash_generic_kernel(FaParams p, int D) {
     for (int e = 0; e < D; ++e) o[e] = (f16)(acc[e] / l);
 }
 
-// Whether the score/output kernel runs its 32-query pairs (128 queries a workgroup) instead of the
-// 64-query ones.  A 64-key block costs a workgroup of 32-query pairs about 0.70 (D > 96) or 0.75
+// The score/output kernel runs 32-query pairs (128 queries a workgroup) or 64-query ones.  A 64-key
+// block costs a workgroup of 32-query pairs about 0.70 (D > 96) or 0.75
 // of what it costs one of 64-query pairs, and a workgroup's start and end about 1.5 such blocks, so
 // twice the workgroups pay where the wide ones leave CUs idle or, causal, the longest of them (its
 // last query block's ceil(S / 64) key blocks) outlasts the rest.  Measured (us, 64- / 32-query pairs;
@@ -1044,16 +1388,23 @@ __global__ void flash_generic_kernel(FaParams p, int D) {
 // H = 8, S = 2048 44.0 / 30.1; B = 2, H = 16, S = 512 16.3 / 11.6; but B = 4, H = 32, S = 512 19.2 /
 // 21.4, 1024 54.8 / 58.2, 4096 504 / 598; H = 4, S = 4096, D = 64 64.0 / 48.0; B = 4, H = 12, S = 777,
 // D = 64 18.1 / 25.9.
-static bool fa_narrow_preferred(int64_t S, int64_t heads, int64_t D, bool causal) {
-    auto cost = [&](int64_t bq, double block) {
-        const double nqb = (double)((S + bq - 1) / bq), nkb = (double)((S + F5_BK - 1) / F5_BK);
-        const double wgs = nqb * (double)heads, per = (double)(bq / F5_BK), rounds = std::ceil(wgs / 256);
-        // key blocks on the busiest CU: causal, a head's sum spread over the CUs, or its longest one
-        const double sum = per * nqb * (nqb + 1) / 2 - (nqb * per - nkb);
-        const double blocks = causal ? std::max(nkb, sum * (double)heads / 256) : rounds * nkb;
-        return block * blocks + 1.5 * rounds;
-    };
-    return cost(32 * F5_PAIRS, D > 96 ? 0.70 : 0.75) < cost(64 * F5_PAIRS, 1.0);
+//
+// flash_fwd6_kernel (D = 56 and 64) takes 0.93 of that block with 64-query groups and 0.58 with 32-query
+// ones, two blocks at a time, and 2.3 and 2.1 for its start and merge: (64-query pairs / 32-query pairs /
+// its two widths) H = 32, B = 4, S = 4096 causal 343 / 445 / 323 / 374; B = 1, H = 32, S = 2500 not causal
+// 87 / 94 / 84 / 77; B = 4, H = 12, S = 777 not causal 18.2 / 26 / 18.7 / 23.1; B = 4, H = 16, S = 300 causal
+// 9.7 / 7.5 / 10.4 / 7.8.
+//
+// The key blocks' time on the busiest CU plus its workgroups' starts and ends, in 64-query-pair blocks;
+// step: key blocks taken at a time.
+static double fa_cost(int64_t S, int64_t heads, bool causal, int64_t bq, double block, double start, int64_t step) {
+    const double nqb = (double)((S + bq - 1) / bq);
+    const double nkb = (double)(((S + F5_BK - 1) / F5_BK + step - 1) / step * step);
+    const double wgs = nqb * (double)heads, per = (double)bq / F5_BK, rounds = std::ceil(wgs / 256);
+    // causal: a head's sum spread over the CUs, or its longest workgroup
+    const double sum = per * nqb * (nqb + 1) / 2 - std::max(0.0, nqb * per - nkb);
+    const double blocks = causal ? std::max(nkb, sum * (double)heads / 256) : rounds * nkb;
+    return block * blocks + start * rounds;
 }
 
 }  // namespace lava
@@ -1126,6 +1477,23 @@ extern "C" int lava_hip_flash_attn_fwd_f16(const void* Q, const void* K, const v
                    aligned(Q, 16) && aligned(K, 16) && aligned(V, 16) && aligned(O, 8) &&
                    S * strides[1] * 2 < ((int64_t)1 << 31);
     for (int i = 1; i < 4; ++i) fast256 = fast256 && strides[i] % 8 == 0 && os[i] % 4 == 0;
+    const double cost5w = fa_cost(S, H * B, p.causal, 64 * F5_PAIRS, 1.0, 1.5, 1);
+    const double cost5n = fa_cost(S, H * B, p.causal, 32 * F5_PAIRS, D > 96 ? 0.70 : 0.75, 1.5, 1);
+    if (fast5 && pin == 0 && D > 48 && D <= 64 && scale > 0.f && p.scale_log2 <= 1.f) {
+        const double cost6w = fa_cost(S, H * B, p.causal, 64 * F6_GROUPS, 0.93, 2.3, 2);
+        const double cost6n = fa_cost(S, H * B, p.causal, 32 * F6_GROUPS, 0.58, 2.1, 2);
+        if (std::min(cost6w, cost6n) < 0.96 * std::min(cost5w, cost5n)) {   // (the estimates hold to a few percent)
+            auto go = [&](auto kernel, int64_t bq) {
+                hipLaunchKernelGGL(kernel, dim3((unsigned)(((S + bq - 1) / bq) * H * B)), dim3(128 * F6_GROUPS), 0, s, p);
+            };
+            if (cost6n < cost6w)
+                p.causal ? go(flash_fwd6_kernel<true, 1>, 32 * F6_GROUPS) : go(flash_fwd6_kernel<false, 1>, 32 * F6_GROUPS);
+            else
+                p.causal ? go(flash_fwd6_kernel<true, 2>, 64 * F6_GROUPS) : go(flash_fwd6_kernel<false, 2>, 64 * F6_GROUPS);
+            LAVA_LAUNCH_CHECK("flash_fwd6_kernel");
+            return LAVA_HIP_OK;
+        }
+    }
     if (fast5) {   // any D <= 128, a multiple of 8 (staged zero-padded to 128; MFMAs over D rounded up to 64, 96, 128)
         auto go = [&](auto kernel, int64_t blocks) {
             hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(128 * F5_PAIRS), 0, s, p);
@@ -1138,7 +1506,7 @@ extern "C" int lava_hip_flash_attn_fwd_f16(const void* Q, const void* K, const v
             else if (D <= 96) go(flash_fwd5_kernel<C, 96, QH>, blocks);
             else go(flash_fwd5_kernel<C, 128, QH>, blocks);
         };
-        const bool narrow = fa_narrow_preferred(S, H * B, D, p.causal);
+        const bool narrow = cost5n < cost5w;
         typedef std::integral_constant<int, 1> Q1;
         typedef std::integral_constant<int, 2> Q2;
         if (p.causal)
