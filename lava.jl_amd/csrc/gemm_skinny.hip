@@ -96,7 +96,7 @@ __global__ void __launch_bounds__(256, 1)
     const int tm = BLONG ? 0 : blockIdx.x, tn = BLONG ? blockIdx.x : 0;
     const int a_rows = (int)min((int64_t)SK_TILE, bnd.m - (int64_t)tm * SK_TILE);
     const int b_rows = (int)min((int64_t)SK_TILE, bnd.n - (int64_t)tn * SK_TILE);
-    const int kelems = bnd.kb / (int)sizeof(T);
+    const int kelems = bnd.kb / (int)sizeof(T), ktiles = (bnd.kb + TN_KB - 1) / TN_KB;
     TnSide<T, AK, SK_TILE> sa;
     TnSide<T, BK, SK_TILE> sb;
     sa.init(A, lda_b, tm, a_rows, bnd.m, kelems, w, 0, lane);
@@ -108,8 +108,10 @@ __global__ void __launch_bounds__(256, 1)
         const uint32_t dst = lds0 + slot * SK_STAGE;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {   // unit q / 2, instruction q % 2
-            const uint32_t kofs = (uint32_t)min(2 * s + (q >> 1), 2 * stages - 1) * TN_KB;
-            const bool live = s < stages;
+            // units past K: no address, and the last unit's offset, so that none leaves 2 GiB
+            const int unit = 2 * s + (q >> 1);
+            const uint32_t kofs = (uint32_t)min(unit, ktiles - 1) * TN_KB;
+            const bool live = unit < ktiles;
             const int i = q & 1;
             const uint32_t va = live && sa.valid(i, kofs, bnd.kb) ? sa.voff(i) : OOB_OFS;
             const uint32_t vb = live && sb.valid(i, kofs, bnd.kb) ? sb.voff(i) : OOB_OFS;
