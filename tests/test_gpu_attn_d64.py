@@ -1,7 +1,8 @@
 """Attention at D = 56 and 64 on the kernel that keeps both products in one wavefront: grids that give its
 64-query groups (many heads) and its 32-query ones (few), an odd and an even number of key blocks, S at
 the edges of a block, scales that keep the running maximum still and that move it, strided rows, O rows
-8-byte aligned.  Reference: softmax in 64 bits; bar: the attention configurations' relative Frobenius
+8-byte aligned.  The wide causal grids near S = 2200 lie within the rule's 4 % margin and keep the score/output
+kernel; those above 4096 leave it.  Reference: softmax in 64 bits; bar: the attention configurations' relative Frobenius
 error of 2e-3 (fp16 probabilities and result, 2^-11 each)."""
 import math
 
@@ -16,7 +17,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("E,L,H,B,scale,pad", [
     (64, 1025, 4, 1, None, 0), (64, 1152, 3, 2, 0.6, 0), (56, 1313, 4, 1, None, 8), (64, 1089, 2, 1, 0.02, 4),
-    (64, 2176, 36, 4, None, 0), (56, 2113, 32, 5, 0.5, 8), (64, 2300, 30, 5, 0.6, 4)])
+    (64, 2176, 36, 4, None, 0), (56, 2113, 32, 5, 0.5, 8), (64, 2300, 30, 5, 0.6, 4),
+    (64, 4161, 32, 4, None, 0), (56, 4480, 30, 5, 0.5, 8), (64, 4607, 28, 5, 0.6, 4)])
 def test_flash_d64_one_wavefront(gpu, E, L, H, B, scale, pad, causal):
     lh = gpu
     announce(f"flash D={E} one wavefront S={L} H={H} B={B} scale={scale} pad={pad} causal={causal}")
@@ -28,7 +30,8 @@ def test_flash_d64_one_wavefront(gpu, E, L, H, B, scale, pad, causal):
     sc = 1 / math.sqrt(E) if scale is None else scale
     lh.kernel_log_clear()
     lh.flash_attn_fwd_raw(Q.ptr, K.ptr, V.ptr, O.ptr, B, H, L, E, Q.strides(), O.strides(), sc, causal)
-    assert lh.kernel_log() == ["flash_fwd6_kernel"], lh.kernel_log()
+    near = causal and 2000 < L < 2400   # estimated at 0.976 to 0.98 of the score/output kernel's time
+    assert lh.kernel_log() == ["flash_fwd5_kernel" if near else "flash_fwd6_kernel"], lh.kernel_log()
     q, k, v, got = (a.to_numpy() for a in (Q, K, V, O))
     assert not np.isnan(got[:E].astype(np.float32)).any()
     assert (np.ascontiguousarray(got[E:]).view(np.uint16) == 0xFFFF).all(), "row padding of O written"
