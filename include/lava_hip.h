@@ -131,7 +131,11 @@ int lava_hip_release_workspaces(void);
 /* ========================================================================= */
 
 /* The names of the kernels this thread launched since its last lava_hip_kernel_log_clear(),
- * '+'-separated, the newest last (at most 255 bytes; the oldest names are dropped first). */
+ * '+'-separated, the newest last (at most 255 bytes; the oldest names are dropped first).  A kernel's
+ * separate form has its own name behind the kernel's: gemm_mid_ksplit_kernel behind gemm_mid_kernel (the
+ * K-split form), gemm_small_kernel<any> behind gemm_small_kernel and gemm_small_kernel<u8,any> behind
+ * gemm_small_kernel<u8> (operands of any alignment), flash_fwd5_kernel<32> and flash_fwd6_kernel<32>
+ * behind the name without <32> (32 queries a wavefront pair or group instead of 64). */
 const char* lava_hip_kernel_log(void);
 void lava_hip_kernel_log_clear(void);
 

@@ -1490,7 +1490,7 @@ extern "C" int lava_hip_flash_attn_fwd_f16(const void* Q, const void* K, const v
                 p.causal ? go(flash_fwd6_kernel<true, 1>, 32 * F6_GROUPS) : go(flash_fwd6_kernel<false, 1>, 32 * F6_GROUPS);
             else
                 p.causal ? go(flash_fwd6_kernel<true, 2>, 64 * F6_GROUPS) : go(flash_fwd6_kernel<false, 2>, 64 * F6_GROUPS);
-            LAVA_LAUNCH_CHECK("flash_fwd6_kernel");
+            LAVA_LAUNCH_CHECK(cost6n < cost6w ? "flash_fwd6_kernel+flash_fwd6_kernel<32>" : "flash_fwd6_kernel");
             return LAVA_HIP_OK;
         }
     }
@@ -1513,7 +1513,7 @@ extern "C" int lava_hip_flash_attn_fwd_f16(const void* Q, const void* K, const v
             narrow ? by_d(f3_tag<true>{}, Q1{}) : by_d(f3_tag<true>{}, Q2{});
         else
             narrow ? by_d(f3_tag<false>{}, Q1{}) : by_d(f3_tag<false>{}, Q2{});
-        LAVA_LAUNCH_CHECK("flash_fwd5_kernel");
+        LAVA_LAUNCH_CHECK(narrow ? "flash_fwd5_kernel+flash_fwd5_kernel<32>" : "flash_fwd5_kernel");
         return LAVA_HIP_OK;
     }
     if (fast3) {

@@ -535,7 +535,8 @@ int launch_small_grid(const T* A, const T* B, OutT* C, int64_t M, int64_t N, int
         by_layout(std::integral_constant<bool, true>{});
     else
         by_layout(std::integral_constant<bool, false>{});
-    LAVA_LAUNCH_CHECK(U8 ? "gemm_small_kernel<u8>" : "gemm_small_kernel");
+    LAVA_LAUNCH_CHECK(any ? (U8 ? "gemm_small_kernel<u8>+gemm_small_kernel<u8,any>" : "gemm_small_kernel+gemm_small_kernel<any>")
+                          : (U8 ? "gemm_small_kernel<u8>" : "gemm_small_kernel"));
     return LAVA_HIP_OK;
 }
 }  // namespace

@@ -268,7 +268,7 @@ int launch_gemm_mid_ksplit(const T* A, const T* B, typename Mfma16<T>::acc_elem*
         else go(gemm_mid_ksplit_kernel<T, R, true, true>);
     };
     ragged ? by_layout(std::true_type{}) : by_layout(std::false_type{});
-    LAVA_LAUNCH_CHECK("gemm_mid_kernel");
+    LAVA_LAUNCH_CHECK("gemm_mid_kernel+gemm_mid_ksplit_kernel");   // a form's name follows its kernel's
     return LAVA_HIP_OK;
 }
 template int launch_gemm_mid_ksplit<f16>(const f16*, const f16*, float*, int64_t, int64_t, int64_t, int64_t, int64_t,

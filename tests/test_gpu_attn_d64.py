@@ -30,8 +30,11 @@ def test_flash_d64_one_wavefront(gpu, E, L, H, B, scale, pad, causal):
     sc = 1 / math.sqrt(E) if scale is None else scale
     lh.kernel_log_clear()
     lh.flash_attn_fwd_raw(Q.ptr, K.ptr, V.ptr, O.ptr, B, H, L, E, Q.strides(), O.strides(), sc, causal)
-    near = causal and 2000 < L < 2400   # estimated at 0.976 to 0.98 of the score/output kernel's time
-    assert lh.kernel_log() == ["flash_fwd5_kernel" if near else "flash_fwd6_kernel"], lh.kernel_log()
+    if causal and 2000 < L < 2400:   # estimated at 0.976 to 0.98 of the score/output kernel's time
+        kernel = ["flash_fwd5_kernel"]
+    else:
+        kernel = ["flash_fwd6_kernel"] if H * B > 100 else ["flash_fwd6_kernel", "flash_fwd6_kernel<32>"]
+    assert lh.kernel_log() == kernel, lh.kernel_log()
     q, k, v, got = (a.to_numpy() for a in (Q, K, V, O))
     assert not np.isnan(got[:E].astype(np.float32)).any()
     assert (np.ascontiguousarray(got[E:]).view(np.uint16) == 0xFFFF).all(), "row padding of O written"

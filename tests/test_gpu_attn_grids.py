@@ -12,6 +12,16 @@ from conftest import announce
 pytestmark = pytest.mark.gpu
 
 
+def _kernel(E, L, heads, causal):
+    """The log of the width that the rule takes: 64-query pairs where many heads fill the CUs with them
+    (a sequence of at most 128 has no use for more than one 128-query workgroup a head), except at D =
+    128 causal where the 321 queries leave a second 256-query workgroup nearly empty."""
+    if E == 64 and heads == 3 and L == 321:   # few heads, more than two key blocks a wavefront
+        return ["flash_fwd6_kernel", "flash_fwd6_kernel<32>"]
+    wide = heads > 256 and L > 128 and not (E == 128 and causal and L == 321)
+    return ["flash_fwd5_kernel"] if wide else ["flash_fwd5_kernel", "flash_fwd5_kernel<32>"]
+
+
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("H,B", [(32, 16), (3, 1)])
 @pytest.mark.parametrize("E", [32, 64, 80, 128])
@@ -26,7 +36,7 @@ def test_flash_both_widths(gpu, E, L, H, B, causal):
     O.fill_bytes(0xFF)
     lh.kernel_log_clear()
     lh.flash_attn_fwd(O, Q, K, V, causal=causal)
-    assert "flash_fwd5_kernel" in lh.kernel_log() or E == 64, lh.kernel_log()
+    assert lh.kernel_log() == _kernel(E, L, H * B, causal), lh.kernel_log()
     got = O.to_numpy()
     assert not np.isnan(got).any()
     for h, b in {(0, 0), (H - 1, B - 1), (H // 2, B // 2)}:
