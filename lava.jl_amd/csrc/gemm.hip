@@ -87,7 +87,7 @@ int gemm_entry(const char* name, const void* A, const void* B, void* C, int64_t 
             if (mfit != TN_NO && pin == 0 && skinny_gemm_preferred(M, N, K * (int64_t)sizeof(T), sizeof(T), arow, !brow))
                 return launch_gemm_skinny<T>(a, b, c, M, N, K, lda, ldb, ldc, s, arow, !brow);
         }
-        const bool ksplit = !EPI && !U8 && mid_ksplit_preferred(M, N, K * (int64_t)sizeof(T));
+        const bool ksplit = !EPI && !U8 && pin == 0 && mid_ksplit_preferred(M, N, K * (int64_t)sizeof(T));
         if (mfit != TN_NO && (pin == 4 || (pin == 0 && (ksplit || mid_gemm_preferred(M, N))))) {
             if constexpr (!EPI && !U8) {
                 if (ksplit)

@@ -78,6 +78,7 @@ def _pinned_gemm(gpu, choice, name):
     finally:
         gpu.set_kernel_override(gpu.FAMILY_GEMM, 0)
     assert name in log, f"expected {name} in the kernel log, got {log}"
+    assert "gemm_mid_ksplit_kernel" not in log, f"pinned to {name}, got {log}"
 
 
 @pytest.fixture

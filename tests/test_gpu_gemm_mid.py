@@ -199,6 +199,26 @@ def test_mid_kernel_repeatable_and_linear(gpu, oracle, mid_kernel):
     np.testing.assert_array_equal(out[0] + out[1], out[2])
 
 
+@pytest.mark.parametrize("dt,shape", [("bf16", (2048, 2048, 2048)), ("f16", (1536, 1536, 4096)),
+                                      ("i8", (2048, 2048, 4096)), ("bf16", (528, 2824, 4168))])
+def test_mid_kernel_pin_is_not_the_ksplit_form(gpu, oracle, mid_kernel, dt, shape):
+    """Choice 4 runs gemm_mid_kernel itself where the automatic choice takes its K-split form, so the two
+    can be told apart and timed against each other; sampled rows against the oracle."""
+    lh = gpu
+    M, N, K = shape
+    announce(f"gemm pinned to the mid-size kernel {dt} M={M} N={N} K={K}")
+    A = lh.HIPDeviceArray(dt, (M, K), order="C")
+    B = lh.HIPDeviceArray(dt, (K, N), order="F")
+    fill(lh, A, dt, 8800 + M)
+    fill(lh, B, dt, 8900 + N)
+    C = lh.HIPDeviceArray("i32" if dt == "i8" else "f32", (M, N), order="C")
+    lh.kernel_log_clear()
+    lh.gemm(C, A, B)
+    assert lh.kernel_log() == ["gemm_mid_kernel"], lh.kernel_log()
+    rows = np.array([0, 1, 127, 128, M // 2, M - 1])
+    check(oracle, dt, C.to_numpy()[rows], A, B, M, N, K, K, K, rows, 1)
+
+
 @pytest.mark.parametrize("dt,shape,kernel,aorder,border",
                          [("bf16", (2048, 2048, 2048), "gemm_mid_kernel", "C", "F"),
                           ("i8", (2048, 4096, 4096), "gemm_mid_kernel", "C", "F"),
