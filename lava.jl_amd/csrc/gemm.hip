@@ -84,7 +84,9 @@ int gemm_entry(const char* name, const void* A, const void* B, void* C, int64_t 
     if constexpr (EPI || std::is_same<OutT, typename Mfma16<T>::acc_elem>::value) {
         const int mfit = mid_gemm_eligible<T>(a, b, c, M, N, K, lda, ldb, ldc, sizeof(OutT), arow, !brow);
         if constexpr (!EPI && !U8) {
-            if (mfit != TN_NO && pin == 0 && skinny_gemm_preferred(M, N, K * (int64_t)sizeof(T), sizeof(T), arow, !brow))
+            const bool lines = M <= 64 ? whole_lines(b, ldb * (int64_t)sizeof(T)) : whole_lines(a, lda * (int64_t)sizeof(T));
+            if (mfit != TN_NO && pin == 0 &&
+                skinny_gemm_preferred(M, N, K * (int64_t)sizeof(T), sizeof(T), arow, !brow, lines))
                 return launch_gemm_skinny<T>(a, b, c, M, N, K, lda, ldb, ldc, s, arow, !brow);
         }
         const bool ksplit = !EPI && !U8 && pin == 0 && mid_ksplit_preferred(M, N, K * (int64_t)sizeof(T));

@@ -93,11 +93,12 @@ int launch_gemm_mid_ksplit(const T* A, const T* B, typename Mfma16<T>::acc_elem*
                            int64_t lda, int64_t ldb, int64_t ldc, hipStream_t s, bool ragged, bool ak, bool bk);
 bool mid_ksplit_preferred(int64_t M, int64_t N, int64_t k_bytes);
 // Products of at most 64 rows or columns on 64 x 64 tiles over all of K (gemm_skinny.hip): the operands
-// and extents of mid_gemm_eligible, int8 with both operands K-contiguous; and whether one runs on it.
+// and extents of mid_gemm_eligible, int8 with both operands K-contiguous; and whether one runs on it
+// (lines: whole_lines of the long operand -- B with at most 64 rows, else A).
 template <typename T>
 int launch_gemm_skinny(const T* A, const T* B, typename Mfma16<T>::acc_elem* C, int64_t M, int64_t N, int64_t K,
                        int64_t lda, int64_t ldb, int64_t ldc, hipStream_t s, bool ak, bool bk);
-bool skinny_gemm_preferred(int64_t M, int64_t N, int64_t k_bytes, size_t elem, bool ak, bool bk);
+bool skinny_gemm_preferred(int64_t M, int64_t N, int64_t k_bytes, size_t elem, bool ak, bool bk, bool lines);
 // Whether an M x N product takes the mid-size kernel when it fits (the measured choice against the
 // tile and small-product kernels).
 bool mid_gemm_preferred(int64_t M, int64_t N);

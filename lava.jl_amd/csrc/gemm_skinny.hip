@@ -240,20 +240,35 @@ template int launch_gemm_skinny<bf16>(const bf16*, const bf16*, float*, int64_t,
 template int launch_gemm_skinny<int8_t>(const int8_t*, const int8_t*, int32_t*, int64_t, int64_t, int64_t, int64_t,
                                         int64_t, int64_t, hipStream_t, bool, bool);
 
-// Measured against the small-product kernel (us, that / this; 64 rows, bf16 unless said):
-//  * from 4096 bytes of K that one splits K, and this one needs about a tile per CU: 14336 x 4096 (224
-//    tiles) 29.2 / 26.9, with W N-contiguous 32.5 / 29.0, 14336 rows x 64 columns 36.9 / 27.2, 16 rows
-//    26.4 / 23.9, 12288 x 4096 (192) 24.8 / 23.0 at 33 rows, int8 15.5 / 14.9, 16384 x 4096 (256) 46.6 /
-//    29.6, int8 20.9 / 17.1; but 11008 (172) 25.1 / 25.5, 4096 (64) 14.1 / 22.1, 28672 (448, a second
-//    round) 53.7 / 57.1, and with 16384 bytes of K 14336 51.8 / 54.0 while 16384 80.1 / 59.5;
-//  * below it does not split: 2048 x 1024 8.5 / 7.6, 512 x 1536 11.3 / 8.4, 8192 x 1024 8.9 / 9.1, 14336 x
-//    1536 13.5 / 12.8; at 1024 bytes (512 x 512) 5.5 / 5.4, 8192 x 512 5.8 / 6.6; int8 at 1024 bytes 1024
-//    columns 5.5 / 5.4, 12288 6.3 / 6.7 (int8 keeps the small-product kernel there).
-bool skinny_gemm_preferred(int64_t M, int64_t N, int64_t k_bytes, size_t elem, bool ak, bool bk) {
-    if ((M < N ? M : N) > SK_TILE || (elem == 1 && !(ak && bk))) return false;
+// Measured against the small-product kernel (us, that / this; the operands resident in the caches between
+// calls, in brackets read from HBM, those of each call elsewhere in 1 GiB; ranges over drawn calls are this one's
+// time over that one's):
+//  * with 192 to 256 tiles (240 above 8192 bytes of K) and a long operand whose rows are whole 128-byte lines,
+//    0.60 to 1.00 (0.49 to 0.98), whether that one splits K or not: 64 x 14336 x 4096 bf16 29.2 / 26.9, W
+//    N-contiguous 32.5 / 29.0, 64 x 16384 x 4096 46.6 / 29.6.  Fewer tiles leave CUs idle, more make a second
+//    round: 11008 (172) 25.1 / 25.5, 4096 (64) 14.1 / 22.1, 28672 (448) 53.7 / 57.1;
+//  * rows that cross lines cost this one more: its units are 128 bytes of K, which then lie in two lines each, that
+//    one's are 512.  Both operands K-contiguous: up to 32 rows 0.60 to 1.17 (0.49 to 1.07), median 0.91; to 48
+//    0.75 to 1.11 (0.59 to 1.05) where that one does not split K, but 0.91 to 1.36 (0.82 to 1.17) where it does; 64 rows
+//    0.76 to 1.52 (0.59 to 1.39): i8 64 x 14400 x 8096 27.9 / 39.0 (31.9 / 38.5), bf16 64 x 15360 x 16200 103.7 /
+//    145.5 (102.4 / 141.9).  One of them M/N-contiguous: 0.71 to 1.15 (0.59 to 1.07) up to 8192 bytes of K, 64
+//    rows above that 0.89 to 1.30 (0.85 to 1.13).  From 255 tiles that kernel gives way to the mid-size one, which
+//    this one leads on any rows (0.54 to 0.97);
+//  * fewer tiles and less than 4096 bytes of K: 0.65 to 0.91 (0.64 to 1.09) while that one does not split K, 1.14
+//    to 1.77 (1.08 to 2.02) where it does: bf16 1344 x 64 x 2024 8.5 / 14.7 (9.6 / 19.3).  Below 2048 bytes of K
+//    0.81 to 1.03 (0.75 to 1.10), int8 at 1024 bytes and 12288 columns 6.3 / 6.7: left to that one.
+bool skinny_gemm_preferred(int64_t M, int64_t N, int64_t k_bytes, size_t elem, bool ak, bool bk, bool lines) {
+    const int64_t few = M < N ? M : N;
+    if (few > SK_TILE || (elem == 1 && !(ak && bk))) return false;
     const int64_t tiles = ((M < N ? N : M) + SK_TILE - 1) / SK_TILE;
-    if (k_bytes < 4096) return elem == 2 && k_bytes >= 2048 && tiles <= 256;
-    return tiles <= 256 && tiles >= (k_bytes <= 8192 ? 192 : 240);
+    const bool splits = k_bytes > (tiles > 128 ? 15 : 7) * 512;   // the small-product kernel would (small_gemm_splits)
+    if (k_bytes < 4096) {
+        if (elem != 2 || k_bytes < 2048 || tiles > 256 || splits) return false;
+        if (tiles <= 128) return true;
+    } else if (tiles > 256 || tiles < (k_bytes <= 8192 ? 192 : 240)) {
+        return false;
+    }
+    return lines || tiles >= 255 || few <= (splits ? 32 : 48) || (!(ak && bk) && k_bytes <= 8192);
 }
 
 }  // namespace lava

@@ -42,6 +42,9 @@ size_t stream_workspace_cap(void* stream);
 void w8a16_release_stream(void* stream);
 
 inline bool aligned(const void* p, size_t a) { return (reinterpret_cast<uintptr_t>(p) % a) == 0; }
+// Whether every row of a matrix (leading dimension in bytes) starts on a 128-byte cache line, so that a
+// 128-byte piece of a row is one line and not two.
+inline bool whole_lines(const void* p, int64_t ld_bytes) { return aligned(p, 128) && ld_bytes % 128 == 0; }
 
 }  // namespace lava
 
