@@ -83,13 +83,13 @@ int gemm_entry(const char* name, const void* A, const void* B, void* C, int64_t 
     // the 128 x 128 mid-size kernel: plain output, the fused epilogue (f16 / bf16) or unsigned bytes
     if constexpr (EPI || std::is_same<OutT, typename Mfma16<T>::acc_elem>::value) {
         const int mfit = mid_gemm_eligible<T>(a, b, c, M, N, K, lda, ldb, ldc, sizeof(OutT), arow, !brow);
+        const bool a_lines = whole_lines(a, lda * (int64_t)sizeof(T)), b_lines = whole_lines(b, ldb * (int64_t)sizeof(T));
         if constexpr (!EPI && !U8) {
-            const bool lines = M <= 64 ? whole_lines(b, ldb * (int64_t)sizeof(T)) : whole_lines(a, lda * (int64_t)sizeof(T));
             if (mfit != TN_NO && pin == 0 &&
-                skinny_gemm_preferred(M, N, K * (int64_t)sizeof(T), sizeof(T), arow, !brow, lines))
+                skinny_gemm_preferred(M, N, K * (int64_t)sizeof(T), sizeof(T), arow, !brow, M <= 64 ? b_lines : a_lines))
                 return launch_gemm_skinny<T>(a, b, c, M, N, K, lda, ldb, ldc, s, arow, !brow);
         }
-        const bool ksplit = !EPI && !U8 && pin == 0 && mid_ksplit_preferred(M, N, K * (int64_t)sizeof(T));
+        const bool ksplit = !EPI && !U8 && pin == 0 && mid_ksplit_preferred(M, N, K * (int64_t)sizeof(T), (arow && !a_lines) + (!brow && !b_lines));
         if (mfit != TN_NO && (pin == 4 || (pin == 0 && (ksplit || mid_gemm_preferred(M, N))))) {
             if constexpr (!EPI && !U8) {
                 if (ksplit)

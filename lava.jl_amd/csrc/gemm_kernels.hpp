@@ -87,11 +87,12 @@ template <typename T, typename OutT, bool EPI, bool U8 = false>
 int launch_gemm_mid(const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
                     int64_t ldc, hipStream_t s, const Epilogue& epi, bool ragged, bool ak, bool bk);
 // The mid-size kernel's K-split form (gemm_mid_ksplit.hip): plain products, the operands and extents
-// of mid_gemm_eligible; and whether an eligible product runs on it (it then leads all the others).
+// of mid_gemm_eligible; and whether an eligible product runs on it (it then leads all the others;
+// crossing: how many operands are K-contiguous without whole_lines).
 template <typename T>
 int launch_gemm_mid_ksplit(const T* A, const T* B, typename Mfma16<T>::acc_elem* C, int64_t M, int64_t N, int64_t K,
                            int64_t lda, int64_t ldb, int64_t ldc, hipStream_t s, bool ragged, bool ak, bool bk);
-bool mid_ksplit_preferred(int64_t M, int64_t N, int64_t k_bytes);
+bool mid_ksplit_preferred(int64_t M, int64_t N, int64_t k_bytes, int crossing);
 // Products of at most 64 rows or columns on 64 x 64 tiles over all of K (gemm_skinny.hip): the operands
 // and extents of mid_gemm_eligible, int8 with both operands K-contiguous; and whether one runs on it
 // (lines: whole_lines of the long operand -- B with at most 64 rows, else A).

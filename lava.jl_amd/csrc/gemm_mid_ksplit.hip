@@ -278,19 +278,24 @@ template int launch_gemm_mid_ksplit<bf16>(const bf16*, const bf16*, float*, int6
 template int launch_gemm_mid_ksplit<int8_t>(const int8_t*, const int8_t*, int32_t*, int64_t, int64_t, int64_t, int64_t,
                                             int64_t, int64_t, hipStream_t, bool, bool, bool);
 
-// Measured against gemm_mid_kernel (128 to 256 tiles; us, that / this): 2048^2 x 1024 bf16 14.4 / 15.0, x
-// 1536 19.6 / 20.4, x 2048 23.8 / 21.5, x 4096 42.2 / 34.7; 1536^2 x 2048 21.6 / 20.0; int8 2048^2 x 2048
-// 14.0 / 15.7, x 4096 23.2 / 22.1, x 8192 41.7 / 35.2 -- from 4096 bytes of K on.  Against the
-// small-product kernel, where that has more than 256 tiles of 64 x 64 and so no K split (65 to 127 of
-// 128 x 128): 512 x 2816 x 4096 bf16 36.7 / 31.3, x 8192 69.5 / 52.4, int8 x 8192 36.9 / 30.9, but 1100 x
-// 1000 x 2048 20.6 / 22.9 -- from 8192 bytes on, and for two extents of 512 at least (128 x 14336 x
-// 4096, a weight stream, 40.8 / 47.6).  Above 256 tiles gemm_mid_kernel has its two workgroups per CU
-// (2048 x 4096 x 4096 56.6 / 67.7).
-bool mid_ksplit_preferred(int64_t M, int64_t N, int64_t k_bytes) {
+// Measured (us, the other kernel / this; the operands resident in the caches between calls, in brackets read from
+// HBM, those of each call elsewhere in 1 GiB; ranges over drawn calls are this one's time over the other's):
+//  * against gemm_mid_kernel (128 to 256 tiles), from 4096 bytes of K 0.64 to 1.03 (0.62 to 0.94): 2048^2 x 2048
+//    bf16 23.8 / 21.5 (29.9 / 25.1), x 4096 42.2 / 34.7, 1536^2 x 2048 21.6 / 20.0; int8 2048^2 x 4096 23.2 / 22.1,
+//    x 8192 41.7 / 35.2; below, 2048^2 x 1024 bf16 14.4 / 15.0, x 1536 19.6 / 20.4, int8 x 2048 14.0 / 15.7;
+//  * against the small-product kernel, where that has more than 256 tiles of 64 x 64 and so no K split (65 to
+//    127 of 128 x 128), from 8192 bytes of K 0.52 to 1.09 (0.65 to 1.20), median 0.82 (0.98): 512 x 2816 x 8192
+//    bf16 69.5 / 52.4 (71.4 / 72.2).  A K-contiguous operand whose rows cross 128-byte lines costs this one more, its
+//    units being 128 bytes of K against that one's 512: one of them 0.88 to 1.06 (1.01 to 1.30) below 12288 bytes of
+//    K, 0.66 to 1.03 (0.86 to 1.37) above; both 0.84 to 1.20 (1.14 to 1.61), f16 512 x 3072 x 11432 104.1 / 109.6
+//    (113.6 / 156.9).  Two extents of 512 at least: 128 x 14336 x 4096, a weight stream, 40.8 / 47.6; 1100 x
+//    1000 x 2048 20.6 / 22.9.
+// Above 256 tiles gemm_mid_kernel has its two workgroups per CU (2048 x 4096 x 4096 56.6 / 67.7).
+bool mid_ksplit_preferred(int64_t M, int64_t N, int64_t k_bytes, int crossing) {
     const int64_t t128 = ((M + TM_TILE - 1) / TM_TILE) * ((N + TM_TILE - 1) / TM_TILE);
     if (t128 > 256) return false;
     if (t128 >= 128) return k_bytes >= 4096;
-    return k_bytes >= 8192 && M >= 512 && N >= 512 && ((M + 63) / 64) * ((N + 63) / 64) > 256;
+    return crossing < 2 && k_bytes >= (crossing ? 12288 : 8192) && M >= 512 && N >= 512 && ((M + 63) / 64) * ((N + 63) / 64) > 256;
 }
 
 }  // namespace lava
