@@ -435,7 +435,8 @@ int lava_hip_gemm_i8_i32(const void* A, const void* B, void* C, int64_t M, int64
  * column sum) + 16384 K back after their last k-step.  The kernel choice is the signed one's
  * (tile kernel, 128 x 128 mid-size kernel, small-product kernel with K split through the
  * per-stream workspace, in their unsigned forms); shapes no MFMA kernel takes (a K-contiguous K or
- * an M/N-contiguous M/N below 16) run on a one-thread-per-element kernel.  Same layouts and leading-dimension rules as above. */
+ * an M/N-contiguous M/N below 16; unaligned K-contiguous operands with K at most 28 and M N small) run
+ * on a one-thread-per-element kernel.  Same layouts and leading-dimension rules as above. */
 int lava_hip_gemm_u8_u32(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda,
                          int64_t ldb, int64_t ldc, uint32_t layout, void* stream);
 

@@ -15,7 +15,8 @@
 // tiles (small_gemm_preferred's rate estimate), take the 64 x 64 small-product kernel (with K
 // split over the stream's workspace where its tiles alone would leave CUs idle:
 // small_gemm_splits); operands that are not 16-byte aligned or whose extents split a 16-byte chunk
-// that kernel's any-alignment form; and the rest (rows shorter than 16 bytes) the staged kernel.
+// that kernel's any-alignment form, unless K is too short to pay (small_any_preferred); and the rest
+// (those, and rows shorter than 16 bytes) the staged kernel.
 // Unsigned bytes (lava_hip_gemm_u8_u32) take the same choice among the kernels' unsigned forms, and a
 // one-thread-per-element kernel where the staged kernel would run.
 #include <hip/hip_runtime.h>
@@ -127,7 +128,8 @@ int gemm_entry(const char* name, const void* A, const void* B, void* C, int64_t 
             return launch_gemm_tn<T, OutT, EPI>(a, b, c, M, N, K, lda, ldb, ldc, s, epi, fit == TN_RAGGED, arow, !brow);
     }
     // operands that split a 16-byte chunk or are not 16-byte aligned
-    if (pin != 3 && small_any_fits<T>(M, N, K, arow, brow)) return run_small(true);
+    if (pin != 3 && small_any_fits<T>(M, N, K, arow, brow) && (pin == 2 || small_any_preferred(M, N, K, sizeof(T), U8, arow, !brow)))
+        return run_small(true);
     if constexpr (U8) {
         LAVA_REQUIRE((M * N + 255) / 256 <= 0x7fffffff, LAVA_HIP_ERR_UNSUPPORTED, "%s: problem too large", name);
         return launch_gemm_u8_generic(reinterpret_cast<const uint8_t*>(a), reinterpret_cast<const uint8_t*>(b),

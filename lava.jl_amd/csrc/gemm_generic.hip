@@ -494,13 +494,25 @@ bool small_gemm_fits(const void* A, const void* B, int64_t M, int64_t N, int64_t
            ((arow || !brow) ? K % EV == 0 : true) && (arow || M % EV == 0) && (!brow || N % EV == 0);
 }
 // The ANY form reads 16 bytes inside each row, so the contiguous extent of each operand holds at
-// least that much; nothing else is asked of it.  It leads the staged kernel wherever it fits (99.4 ->
-// 17.1 us at 1111 x 1333 x 777); the aligned forms lead it, so it runs where none of them fits.
+// least that much; nothing else is asked of it.  The aligned forms lead it, so it runs where none of them fits.
 template <typename T>
 bool small_any_fits(int64_t M, int64_t N, int64_t K, bool arow, bool brow) {
     constexpr int64_t EV = 16 / (int64_t)sizeof(T);
     if ((M + 63) / 64 > 65535 || (N + 63) / 64 > 0x7fffffff) return false;
     return ((arow || !brow) ? K >= EV : K > 0) && (arow || M >= EV) && (!brow || N >= EV);
+}
+// It leads the staged kernel (99.4 -> 17.1 us at 1111 x 1333 x 777) from two of that one's 64-byte slices of K on.
+// Within one that kernel has no second load latency to wait for, but loads element by element.  Measured over
+// drawn calls, this one's time over that one's (operands resident in the caches between calls, in brackets read
+// from HBM): 16-bit, one slice, above 256 tiles, where that one's smaller workgroups overlap, 0.99 to 1.46 (0.72 to
+// 1.17), median 1.21 (0.93); up to 256 tiles 0.93 to 1.25 (0.60 to 1.03), median 1.05 (0.78); two slices 0.71 to
+// 1.18 (0.44 to 1.05).  Int8 at one slice 0.67 to 1.15 (0.40 to 0.92).  Unsigned bytes against one thread per
+// element, up to 64 tiles: both operands K-contiguous 1.13 to 1.40 (1.06 to 1.31) up to 28 k, 0.60 to 1.14 (0.59
+// to 1.08) to 40; else 0.65 to 1.29 (0.42 to 1.24), median 0.95 (0.70); above 64 tiles 0.12 to 1.07.
+bool small_any_preferred(int64_t M, int64_t N, int64_t K, size_t elem, bool u8, bool ak, bool bk) {
+    const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64);
+    if (u8) return tiles > 64 || K > 28 || !(ak && bk);
+    return elem == 1 || K > 32 || tiles <= 256;
 }
 #define LAVA_SMALL_RULE_INST(T)                                                                                      \
     template bool small_gemm_preferred<T>(int64_t, int64_t, int64_t);                                           \

@@ -24,9 +24,11 @@ template <typename T>
 bool small_gemm_fits(const void* A, const void* B, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, bool arow,
                      bool brow);
 // The kernel's ANY form (any alignment, leading dimension and extent; `any` of the launchers below):
-// whether every row it reads along holds a 16-byte chunk.
+// whether every row it reads along holds a 16-byte chunk; and whether it leads the staged kernel (unsigned
+// bytes: the one-thread-per-element kernel) where it fits.
 template <typename T>
 bool small_any_fits(int64_t M, int64_t N, int64_t K, bool arow, bool brow);
+bool small_any_preferred(int64_t M, int64_t N, int64_t K, size_t elem, bool u8, bool ak, bool bk);
 template <typename T, typename OutT, bool EPI>
 int launch_gemm_small(const T* A, const T* B, OutT* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
                       int64_t ldc, bool arow, bool brow, hipStream_t s, const Epilogue& epi, bool any);

@@ -1,6 +1,8 @@
 """GEMM operands of any alignment, leading dimension and extent, on the kernels' any-alignment forms:
 rows that start at every byte (element) of a 16-byte chunk, K, M and N that split one, K ranges of the
-split product, and nothing read past a row's end (the padding holds NaN, or 255 for the integers).
+split product, and nothing read past a row's end (the padding holds NaN, or 255 for the integers).  A K too
+short for the automatic choice to take unsigned bytes there runs with the small-product kernel pinned; and the
+products on both sides of that rule.
 Reference: numpy in 64 bits.  Floating tolerance: fp32 sums of K terms, each step's relative rounding
 at most 2^-23, random over the terms: sqrt(K) 2^-23 (7.7e-6 at the largest K here)."""
 import math
@@ -40,11 +42,33 @@ def _operand(lh, rng, dt, rows, cols, row_major, pad, shift):
     return dev, dev.pointer(1 + shift), ld, wide if row_major else wide.T
 
 
+@pytest.fixture
+def pin_gemm(gpu):
+    yield lambda choice: gpu.set_kernel_override(gpu.FAMILY_GEMM, choice)
+    gpu.set_kernel_override(gpu.FAMILY_GEMM, 0)
+
+
 @pytest.mark.parametrize("layout", range(8))
 @pytest.mark.parametrize("dt", ["f16", "bf16", "i8", "u8"])
 @pytest.mark.parametrize("shape", [(16, 16, 16), (17, 31, 23), (64, 65, 257), (129, 63, 513), (70, 33, 4099)])
-def test_gemm_any_alignment(gpu, dt, layout, shape):
-    lh = gpu
+def test_gemm_any_alignment(gpu, pin_gemm, dt, layout, shape):
+    if dt == "u8" and shape[2] <= 28:
+        pin_gemm(2)
+    _run(gpu, dt, layout, shape, "gemm_small_kernel<u8,any>" if dt == "u8" else "gemm_small_kernel<any>")
+
+
+@pytest.mark.parametrize("dt,layout,shape,kernel", [
+    ("f16", 5, (1025, 1031, 32), "gemm_staged_kernel"), ("f16", 5, (1025, 1031, 33), "gemm_small_kernel<any>"),
+    ("bf16", 2, (1025, 1031, 17), "gemm_staged_kernel"), ("bf16", 0, (1019, 1023, 31), "gemm_small_kernel<any>"),
+    ("i8", 5, (1025, 1031, 17), "gemm_small_kernel<any>"), ("u8", 5, (50, 70, 28), "gemm_u8_generic_kernel"),
+    ("u8", 1, (510, 509, 17), "gemm_u8_generic_kernel"), ("u8", 5, (50, 70, 29), "gemm_small_kernel<u8,any>"),
+    ("u8", 7, (50, 70, 20), "gemm_small_kernel<u8,any>"), ("u8", 1, (520, 520, 17), "gemm_small_kernel<u8,any>")])
+def test_gemm_any_short_k(gpu, dt, layout, shape, kernel):
+    """The automatic choice on both sides of its bounds on K and on the tiles."""
+    _run(gpu, dt, layout, shape, kernel)
+
+
+def _run(lh, dt, layout, shape, kernel):
     M, N, K = shape
     for pad, shift in ((0, 0), (1, 1), (3, 5)):
         announce(f"gemm any {dt} layout={layout} M={M} N={N} K={K} pad={pad} shift={shift}")
@@ -58,7 +82,7 @@ def test_gemm_any_alignment(gpu, dt, layout, shape):
         lh.kernel_log_clear()
         lh.gemm_raw(dt, ACC[dt], pa, pb, C.ptr, M, N, K, lda, ldb, ldc, layout)
         if pad:
-            assert ("gemm_small_kernel<u8,any>" if dt == "u8" else "gemm_small_kernel<any>") in lh.kernel_log(), lh.kernel_log()
+            assert kernel in lh.kernel_log(), lh.kernel_log()
         got = C.to_numpy().T
         inner = N if crow else M
         assert (got[:, inner:].copy().view(np.uint8) == 0xEE).all(), "C's padding was written"
