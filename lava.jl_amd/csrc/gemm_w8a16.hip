@@ -573,14 +573,23 @@ static W8Plan plan_w8a16(const void* X, const void* W, int64_t M, int64_t N, int
         p.mb = M <= 16 ? 1 : (M <= 32 ? 2 : 4);
         while (p.mb > 1 && p.xrow && 32 * p.mb * p.kldx >= (int64_t(1) << 32)) p.mb /= 2;
         p.mblocks = (M + 16 * p.mb - 1) / (16 * p.mb);
-        // Batches: the tiled kernel once the streaming one would need more than 256 workgroups (a
-        // second one per CU), measured at K = 4096 (us, streaming / tiled): 72 x 5120 20.4 / 19.2, 192
-        // x 3072 22.6 / 19.8, 128 x 8192 25.3 / 20.1, 256 x 14336 89.0 / 33.4, but 128 x 4096 (256
-        // workgroups) 17.0 / 20.1 and 256 x 2048 16.7 / 19.6.  At most 64 rows stay a weight stream
-        // (one workgroup per 32 columns, 64 x 14336 23.9 / 20.6).  The tile is 128 x 64 or 128 x 128 by
-        // the time of its rounds over the 256 CUs, about 0.55 and 0.85 us per 128 k each: 256 x 8192
-        // (256 and 128 tiles) 27.1 / 31.6, 256 x 11008 (344 and 172) 41.5 / 33.3.
-        if (M > 64 && p.cblocks * p.mblocks > 256 && w8a16_batch_fits(M, N, p.kldx, K, ldw, p.xrow)) {
+        // Batches: the tiled kernel once the streaming one would need more than two workgroups per CU, or more
+        // than one and K pays for the tiled one's longer start and four-way merge (about 6 us against 4).
+        // Measured over drawn calls, K 256 to 14336, tiled over streaming (weights resident in the caches
+        // between calls, in brackets read from HBM): above 512 workgroups 0.17 to 0.95 (0.20 to 0.95) but for
+        // one of 42 calls with K below 512, 1.10 (1.11); 257 to 512, X row-major or copied, 1.04 to 1.51 (1.03 to
+        // 1.55) below 1024 k, 0.90 to 1.15 (0.92 to 1.37) below 1536, 0.65 to 1.04 (0.89 to 1.31, median 1.03)
+        // from there on; X column-major 0.89 to 1.32 (0.86 to 1.30) below 1024 k, 0.41 to 0.95 (0.54 to 1.03)
+        // from there on.  At K = 4096 (us, streaming / tiled): 72 x 5120 19.5 / 19.0 (21.0 / 21.1), 192 x 3072
+        // 20.3 / 19.8 (23.2 / 25.7), 128 x 8192 23.2 / 21.3 (25.0 / 27.2), 256 x 14336 91.6 / 37.4 (93.3 / 39.0), but
+        // 128 x 4096 (256 workgroups) 17.0 / 20.1 and 256 x 2048 16.7 / 19.6.  At most 64 rows stay a weight
+        // stream (one workgroup per 32 columns, 64 x 14336 23.9 / 20.6).  The tile is 128 x 64 or 128 x 128 by
+        // the time of its rounds over the 256 CUs, about 0.55 and 0.85 us per 128 k each, the shorter one in
+        // all but 4 of 282 calls above 512 workgroups (those at most 1.13 of the other): 256 x 8192 (256 and 128
+        // tiles) 27.1 / 31.6, 256 x 11008 (344 and 172) 41.5 / 33.3.
+        const int64_t wgs = p.cblocks * p.mblocks;
+        if (M > 64 && wgs > 256 && (wgs > 512 || K >= (p.xrow ? 1536 : 1024)) &&
+            w8a16_batch_fits(M, N, p.kldx, K, ldw, p.xrow)) {
             const int64_t mt = (M + 127) / 128;
             const int64_t rounds64 = (mt * ((N + 63) / 64) + 255) / 256, rounds128 = (mt * ((N + 127) / 128) + 255) / 256;
             p.bn = 11 * rounds64 > 17 * rounds128 ? 128 : 64;
