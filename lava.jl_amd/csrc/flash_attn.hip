@@ -1387,7 +1387,9 @@ __global__ void flash_generic_kernel(FaParams p, int D) {
 // causal but for the last two): B = 1, H = 32, S = 1537, D = 128 37.8 / 29.4; S = 2048 49.3 / 41.3;
 // H = 8, S = 2048 44.0 / 30.1; B = 2, H = 16, S = 512 16.3 / 11.6; but B = 4, H = 32, S = 512 19.2 /
 // 21.4, 1024 54.8 / 58.2, 4096 504 / 598; H = 4, S = 4096, D = 64 64.0 / 48.0; B = 4, H = 12, S = 777,
-// D = 64 18.1 / 25.9.
+// D = 64 18.1 / 25.9.  Over 800 drawn calls the narrow pairs took 0.62 to 1.03 of the wide ones' time where they
+// are estimated below 0.95 of it, 1.00 to 1.10 from there to 1 (B = 3, H = 16, S = 1300, D = 32 26.0 / 28.6; H = 32, B = 4,
+// S = 380, D = 128 16.2 / 17.3), 0.93 to 1.49 above: so they need an estimate below 0.95.
 //
 // flash_fwd6_kernel (D = 56 and 64) takes 0.93 of that block with 64-query groups and 0.58 with 32-query
 // ones, two blocks at a time, and 2.3 and 2.1 for its start and merge: (64-query pairs / 32-query pairs /
@@ -1506,7 +1508,7 @@ extern "C" int lava_hip_flash_attn_fwd_f16(const void* Q, const void* K, const v
             else if (D <= 96) go(flash_fwd5_kernel<C, 96, QH>, blocks);
             else go(flash_fwd5_kernel<C, 128, QH>, blocks);
         };
-        const bool narrow = cost5n < cost5w;
+        const bool narrow = cost5n < 0.95 * cost5w;
         typedef std::integral_constant<int, 1> Q1;
         typedef std::integral_constant<int, 2> Q2;
         if (p.causal)

@@ -12,14 +12,23 @@ from conftest import announce
 pytestmark = pytest.mark.gpu
 
 
-def _kernel(E, L, heads, causal):
+def _kernel(E, L, heads):
     """The log of the width that the rule takes: 64-query pairs where many heads fill the CUs with them
-    (a sequence of at most 128 has no use for more than one 128-query workgroup a head), except at D =
-    128 causal where the 321 queries leave a second 256-query workgroup nearly empty."""
+    (a sequence of at most 128 has no use for more than one 128-query workgroup a head)."""
     if E == 64 and heads == 3 and L == 321:   # few heads, more than two key blocks a wavefront
         return ["flash_fwd6_kernel", "flash_fwd6_kernel<32>"]
-    wide = heads > 256 and L > 128 and not (E == 128 and causal and L == 321)
+    wide = heads > 256 and L > 128
     return ["flash_fwd5_kernel"] if wide else ["flash_fwd5_kernel", "flash_fwd5_kernel<32>"]
+
+
+@pytest.mark.parametrize("E,L,H,B,kernel", [
+    (32, 1300, 16, 3, ["flash_fwd5_kernel"]), (128, 380, 32, 4, ["flash_fwd5_kernel"]),
+    (80, 1289, 16, 3, ["flash_fwd5_kernel"]), (128, 1537, 32, 1, ["flash_fwd5_kernel", "flash_fwd5_kernel<32>"]),
+    (96, 513, 16, 2, ["flash_fwd5_kernel", "flash_fwd5_kernel<32>"])])
+def test_flash_width_near_the_rule(gpu, E, L, H, B, kernel):
+    """Causal grids on both sides of the margin: estimated at 0.95 to 0.96 of the wide pairs' time, and well
+    below it."""
+    _run(gpu, E, L, H, B, True, kernel)
 
 
 @pytest.mark.parametrize("causal", [True, False])
@@ -27,7 +36,10 @@ def _kernel(E, L, heads, causal):
 @pytest.mark.parametrize("E", [32, 64, 80, 128])
 @pytest.mark.parametrize("L", [1, 33, 64, 97, 129, 192, 256, 321])
 def test_flash_both_widths(gpu, E, L, H, B, causal):
-    lh = gpu
+    _run(gpu, E, L, H, B, causal, _kernel(E, L, H * B))
+
+
+def _run(lh, E, L, H, B, causal, kernel):
     announce(f"flash widths D={E} S={L} H={H} B={B} causal={causal}")
     rng = np.random.default_rng(E + L + H)
     q, k, v = (np.asfortranarray(rng.standard_normal((E, L, H, B)).astype(np.float16)) for _ in range(3))
@@ -36,7 +48,7 @@ def test_flash_both_widths(gpu, E, L, H, B, causal):
     O.fill_bytes(0xFF)
     lh.kernel_log_clear()
     lh.flash_attn_fwd(O, Q, K, V, causal=causal)
-    assert lh.kernel_log() == _kernel(E, L, H * B, causal), lh.kernel_log()
+    assert lh.kernel_log() == kernel, lh.kernel_log()
     got = O.to_numpy()
     assert not np.isnan(got).any()
     for h, b in {(0, 0), (H - 1, B - 1), (H // 2, B // 2)}:
