@@ -15,8 +15,8 @@ void set_error(const char* fmt, ...) __attribute__((format(printf, 1, 2)));
 void clear_error();
 int hip_fail(hipError_t e, const char* what);
 // Launch check: the error (if any) hipGetLastError reports for the launch just made; a launch
-// that succeeded is appended to the thread's kernel log (lava_hip_kernel_log); a kernel's separate
-// form as "kernel+form".
+// that succeeded is appended to the thread's kernel log (lava_hip_kernel_log), which keeps the pointer: a
+// string literal, a kernel's separate form as "kernel+form".
 int check_launch(const char* kernel);
 // The kernel choice pinned for a family (LAVA_HIP_FAMILY_*) by lava_hip_set_kernel_override; 0 = automatic.
 int kernel_override(int family);

@@ -31,24 +31,38 @@ int hip_fail(hipError_t e, const char* what) {
     return e == hipErrorNoDevice ? LAVA_HIP_ERR_NO_DEVICE : LAVA_HIP_ERR_HIP;
 }
 
-// Names of the kernels this thread launched, '+'-separated, the newest last (lava_hip_kernel_log).
+// The kernels this thread launched last (string literals, a ring) and the text lava_hip_kernel_log makes of
+// them: a launch stores a pointer, since some calls are bound by their host time.
+constexpr unsigned KLOG_RING = 128;   // more names than 255 characters hold
+static thread_local const char* g_klaunch[KLOG_RING];
+static thread_local unsigned g_klaunched = 0;   // since the last clear
 static thread_local char g_klog[256] = "";
 
-static void log_kernel(const char* name) {
-    const size_t m = strlen(name);
-    if (m + 1 >= sizeof(g_klog)) return;
-    size_t n = strlen(g_klog);
-    while (n > 0 && n + 1 + m + 1 > sizeof(g_klog)) {   // drop the oldest names until this one fits
-        const char* plus = strchr(g_klog, '+');
-        if (plus == nullptr) {
-            n = 0;
-            break;
+static void log_kernel(const char* name) { g_klaunch[g_klaunched++ % KLOG_RING] = name; }
+
+// '+'-separated, the newest last; the oldest names that do not fit are left out
+static const char* klog_text() {
+    size_t at = sizeof(g_klog) - 1;   // filled from its end
+    g_klog[at] = 0;
+    const unsigned kept = g_klaunched < KLOG_RING ? g_klaunched : KLOG_RING;
+    for (unsigned i = 1; i <= kept; ++i) {
+        const char* name = g_klaunch[(g_klaunched - i) % KLOG_RING];
+        const size_t sep = i > 1 ? 1 : 0;
+        bool whole = true;
+        while (name != nullptr && strlen(name) + sep > at) {   // "kernel+form": the form alone if only it fits
+            name = strchr(name, '+');
+            name = name ? name + 1 : nullptr;
+            whole = false;
         }
-        memmove(g_klog, plus + 1, strlen(plus + 1) + 1);
-        n = strlen(g_klog);
+        if (name != nullptr) {
+            if (sep) g_klog[--at] = '+';
+            const size_t m = strlen(name);
+            at -= m;
+            memcpy(g_klog + at, name, m);
+        }
+        if (!whole) break;
     }
-    if (n > 0) g_klog[n++] = '+';
-    memcpy(g_klog + n, name, m + 1);
+    return g_klog + at;
 }
 
 int check_launch(const char* kernel) {
@@ -206,9 +220,9 @@ extern "C" {
 
 const char* lava_hip_last_error(void) { return g_err; }
 
-const char* lava_hip_kernel_log(void) { return g_klog; }
+const char* lava_hip_kernel_log(void) { return klog_text(); }
 
-void lava_hip_kernel_log_clear(void) { g_klog[0] = 0; }
+void lava_hip_kernel_log_clear(void) { g_klaunched = 0; }
 
 int lava_hip_set_kernel_override(int family, int choice) {
     const bool ok = (family == LAVA_HIP_FAMILY_ATTN && (choice == 0 || choice == 3 || choice == 5)) ||

@@ -76,3 +76,29 @@ def test_mfma_loop_rejects_bad_arguments(gpu):
             lh._lib.call("lava_hip_mfma_loop", *args, sink.ptr, None)
     with pytest.raises(lh.InvalidArgument):
         lh._lib.call("lava_hip_mfma_loop", 0, a.ptr, a.ptr, 4096, 1, 1, 1, C.c_void_p(None), None)
+
+
+def test_kernel_log_keeps_the_newest_names(gpu):
+    """Whole names up to 255 characters, the newest last, however many were launched; a form's name stays when
+    its kernel's no longer fits; clearing forgets them all."""
+    lh = gpu
+    announce("kernel log")
+    A = lh.HIPDeviceArray("f16", (16, 24), order="C")
+    B = lh.HIPDeviceArray("f16", (24, 16), order="C")
+    C = lh.HIPDeviceArray("f32", (16, 16), order="C")
+    odd = lambda: lh.gemm_raw("f16", "f32", A.ptr, B.ptr, C.ptr, 15, 15, 23, 24, 16, 16, 7)
+    lh.kernel_log_clear()
+    assert lh.kernel_log() == []
+    for n in range(1, 300):
+        odd()
+        log = lh.kernel_log()
+        assert len("+".join(log)) <= 255
+        want = ["gemm_small_kernel", "gemm_small_kernel<any>"] * n   # 17 and 22 characters: 6 pairs are 245
+        assert log == want[-12:], (n, log)
+    C.fill_bytes(0)
+    log = lh.kernel_log()
+    assert log[-1] == "fill_bytes_kernel" and log[:-1] == (want * 2)[-11:], log
+    lh.kernel_log_clear()
+    assert lh.kernel_log() == []
+    odd()
+    assert lh.kernel_log() == ["gemm_small_kernel", "gemm_small_kernel<any>"]
