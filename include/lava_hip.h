@@ -104,9 +104,9 @@ int lava_hip_event_elapsed_ms(float* ms, void* start, void* stop);
 /* HIP graphs of the library's calls (thin wrappers over hipStreamBeginCapture in global mode,
  * hipStreamEndCapture + hipGraphInstantiate, hipGraphLaunch, hipGraphExecDestroy): what a caller
  * that replays a fixed sequence of launches uses instead of a tracing compiler.  While a stream
- * captures in global mode, an allocating call anywhere in the process fails; the compute entry
- * points then plan within the workspace the stream already has (lava_hip_gemm_w8a16) or take
- * lava_hip_gemm_w8a16_noalloc.  The NULL stream cannot be captured. */
+ * captures in global mode, lava_hip_malloc fails anywhere in the process; the compute entry points on
+ * that stream plan within the workspace it already has (or take lava_hip_gemm_w8a16_noalloc), on
+ * others they may still allocate theirs.  The NULL stream cannot be captured. */
 int lava_hip_graph_capture_begin(void* stream);
 int lava_hip_graph_capture_end(void* stream, void** exec);
 int lava_hip_graph_launch(void* exec, void* stream);

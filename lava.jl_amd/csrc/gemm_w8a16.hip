@@ -734,7 +734,7 @@ static int check_w8a16_args(const void* X, const void* W, const void* scale, con
 // work already enqueued may still use it -- and every buffer of a stream is freed by
 // lava_hip_stream_destroy (after the stream drains) or lava_hip_release_workspaces (after the
 // device drains).  A stream that is capturing a graph never allocates (hipMalloc is not
-// capturable): its calls plan within the buffer it has (stream_workspace_cap), and that buffer
+// capturable; calls on other streams do, while it captures): its calls plan within the buffer it has (stream_workspace_cap), and that buffer
 // is marked as held by a graph, which may replay it after the stream is gone, so it is moved
 // to g_ws_kept instead of being freed.
 struct W8Workspace {
@@ -780,7 +780,14 @@ int with_stream_workspace(size_t bytes, void* stream, const std::function<int(vo
                      "the stream is capturing a graph and its workspace (%zu bytes) is smaller than this call needs "
                      "(%zu bytes): make one call of this shape outside capture first", ws.bytes, bytes);
         void* buf = nullptr;
-        LAVA_HIP_TRY(hipMalloc(&buf, bytes));
+        // this stream does not capture: its allocation neither waits for nor disturbs one that does, so the
+        // thread's capture mode is relaxed for it (in global mode any other stream's capture would refuse
+        // it and be broken by it)
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        LAVA_HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
+        const hipError_t e = hipMalloc(&buf, bytes);
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+        LAVA_HIP_TRY(e);
         // the W8A16 arrival counters start at zero (every call leaves them at zero)
         const int rc = lava_hip_fill_bytes(buf, 0, STREAM_WS_RESERVED, stream);
         if (rc != LAVA_HIP_OK) {

@@ -128,6 +128,43 @@ def test_splitk_gemm_under_capture_runs_unsplit(gpu, oracle, dt):
     st.close()
 
 
+@pytest.mark.parametrize("lda,kernel", [(4100, "gemm_small_kernel<any>"), (4112, "gemm_small_kernel")])
+def test_workspace_of_a_stream_beside_a_capture(gpu, lda, kernel):
+    """A product that splits K, on a fresh stream while another one captures a graph in global mode: its
+    workspace is allocated all the same and the capture is not disturbed.  (With operands of any
+    alignment the product took no workspace before it had a K split.)"""
+    lh = gpu
+    M, N, K = 70, 48, 4096
+    announce(f"split-K product beside a capture, lda={lda}")
+    A = lh.HIPDeviceArray("f16", (M, lda), order="C")
+    B = lh.HIPDeviceArray("f16", (K, N), order="C")
+    lh.fill_uniform(A, lh_mod.seed(60, 0), -1.0, 1.0)
+    lh.fill_uniform(B, lh_mod.seed(60, 1), -1.0, 1.0)
+    C = lh.HIPDeviceArray("f32", (M, N), order="C")
+    D = lh.HIPDeviceArray("u8", (64,))
+    D.fill_bytes(0)
+    capturing, other = lh.Stream(), lh.Stream()
+    g = lh.Graph(capturing)
+    lh.synchronize()
+    lh.kernel_log_clear()
+    with g.capture():
+        lh._lib.call("lava_hip_fill_bytes", D.ptr, 7, 64, capturing.handle)
+        lh.gemm_raw("f16", "f32", A.ptr, B.ptr, C.ptr, M, N, K, lda, N, N, 7, other.handle)
+    assert kernel in lh.kernel_log() and "splitk_sum_kernel" in lh.kernel_log(), lh.kernel_log()
+    other.synchronize()
+    want = A.to_numpy()[:, :K].astype(np.float64) @ B.to_numpy().astype(np.float64)
+    assert np.linalg.norm(C.to_numpy() - want) <= 64 * 2.0 ** -23 * np.linalg.norm(want)   # sqrt(K) 2^-23
+    for _ in range(2):
+        D.fill_bytes(0)
+        lh.synchronize()
+        g.launch()
+        capturing.synchronize()
+        assert (D.to_numpy() == 7).all()
+    g.close()
+    capturing.close()
+    other.close()
+
+
 def test_release_workspaces(gpu, oracle):
     """The NULL stream's workspaces (split-K GEMM and W8A16) are freed by
     lava_hip_release_workspaces; the next calls allocate them again and give the same bits."""
