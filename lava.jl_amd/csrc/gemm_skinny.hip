@@ -2,11 +2,13 @@
 // 64 x 64 tile of C per workgroup over all of K, f16 / bf16 / int8, plain output.
 //
 // Such a product is bound by reading its long operand (the weights) once: 117 MB at 64 x 14336 x 4096
-// bf16, 18 to 23 us at what HBM streams (26.9 us a call here, 29.2 on the small-product kernel; 23.9 at 16
-// rows, so the short operand's L2 traffic, as many bytes again at 64 rows, is what is left).  The small-product kernel keeps one K chunk per operand in
-// flight in registers, splits K in two to fill the chip and adds the parts in a second kernel; here
-// the loads go straight to LDS and four stages of 32 KB are in flight per CU, so one workgroup per CU
-// streams at the rate of HBM and K needs no split from about one tile per CU on:
+// bf16, 18 to 23 us at what HBM streams.  26.6 us a call here (4.4 TB/s), whether the weights come from HBM (every
+// call's elsewhere in 1 GiB) or lie in the last-level cache from the call before, 23.0 at 16 rows (23.2
+// from HBM), so the short operand's L2 traffic, as many bytes again at 64 rows, is what is left.  The
+// small-product kernel, 27.7 to 29.9 us resident and 30.6 from HBM (16 rows 23.9 and 27.4), keeps one K chunk per
+// operand in flight in registers, splits K in two to fill the chip and adds the parts in a second kernel;
+// here the loads go straight to LDS and four stages of 32 KB are in flight per CU, so one workgroup per CU
+// hides HBM's latency and K needs no split from about one tile per CU on:
 //  * 4 wavefronts, each all of the tile (4 x 4 accumulators) over one 64-byte k-step of every 256 bytes
 //    of K, summed through LDS at the end in a fixed order;
 //  * a stage is 256 bytes of K: two units of 128 bytes (TnSide at 64 rows), A and B, 8 KB each; a ring
