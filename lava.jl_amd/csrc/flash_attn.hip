@@ -1124,10 +1124,12 @@ __global__ void __launch_bounds__(512, 1) flash_fwd6_kernel(FaParams p) {
         for (int qh = 0; qh < QH; ++qh)
 #pragma unroll
             for (int r = 0; r < 16; ++r) o[dt][qh][r] = 0.f;
-    float m_run[QH], l_run[QH];
+    // m is unset (-inf, and 0 taken off the scores) until a block holds a score above -inf; up_at: a score above
+    // it moves m
+    float m_run[QH], l_run[QH], up_at[QH];
 #pragma unroll
     for (int qh = 0; qh < QH; ++qh) {
-        m_run[qh] = 0.f;
+        m_run[qh] = up_at[qh] = -INFINITY;
         l_run[qh] = 0.f;
     }
     const f5_h2 ones = {(_Float16)1.f, (_Float16)1.f};
@@ -1142,7 +1144,7 @@ __global__ void __launch_bounds__(512, 1) flash_fwd6_kernel(FaParams p) {
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) fa_scale_f16(qf[qh][ks], p.scale_log2);
 
-    auto block = [&](int kb, uint32_t st_ofs, bool first) __attribute__((always_inline)) {
+    auto block = [&](int kb, uint32_t st_ofs) __attribute__((always_inline)) {
         f32x16 st[2][QH];   // S' = c q.k - m; st[kt][qh] register r: key 32 kt + 8 (r / 4) + 4 h + r % 4
         auto kread = [&](int f) __attribute__((always_inline)) -> f16x8 {   // f = 2 ks + kt
             return *(const lds_f16x8*)(uintptr_t)(k_rd[f >> 1] + st_ofs + (uint32_t)((f & 1) * 32 * RB));
@@ -1185,7 +1187,7 @@ __global__ void __launch_bounds__(512, 1) flash_fwd6_kernel(FaParams p) {
                     }
         }
         float vl[QH];   // this lane's largest S' per query half
-        bool up = first;
+        bool up = false;
 #pragma unroll
         for (int qh = 0; qh < QH; ++qh) {
             float v = -INFINITY;
@@ -1194,22 +1196,25 @@ __global__ void __launch_bounds__(512, 1) flash_fwd6_kernel(FaParams p) {
 #pragma unroll
                 for (int r = 0; r < 16; ++r) v = fmaxf(v, st[kt][qh][r]);
             vl[qh] = v;
-            up = up || v > F3_RESCALE;
+            up = up || v > up_at[qh];
         }
         if (__builtin_amdgcn_ballot_w64(up) != 0) {
 #pragma unroll
             for (int qh = 0; qh < QH; ++qh) {
                 float a, b;
                 f5_xor32_pair(vl[qh], a, b);
-                // the first block sets m to its maximum (finite: a block's first key is never masked),
-                // later ones only raise it
-                const float t = fmaxf(a, b), d = first ? t : fmaxf(t, 0.f);
-                const float alpha = first ? 1.f : __builtin_amdgcn_exp2f(-d);
-                m_run[qh] += d;
+                // a query's first block with a score above -inf sets m to its maximum, later ones only raise
+                // it; a block of -inf before that (keys masked by infinite operands) leaves it unset
+                const bool set = m_run[qh] != -INFINITY;
+                const float t = fmaxf(a, b), d = set ? fmaxf(t, 0.f) : (t == -INFINITY ? 0.f : t);
+                const float alpha = set ? __builtin_amdgcn_exp2f(-d) : 1.f;
+                m_run[qh] = set ? m_run[qh] + d : t;
+                const bool now_set = m_run[qh] != -INFINITY;
+                up_at[qh] = now_set ? F3_RESCALE : -INFINITY;
                 l_run[qh] *= alpha;
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    neg_m[qh][r] = -m_run[qh];
+                    neg_m[qh][r] = now_set ? -m_run[qh] : 0.f;
                     st[0][qh][r] -= d;
                     st[1][qh][r] -= d;
                     o[0][qh][r] *= alpha;
@@ -1255,7 +1260,7 @@ __global__ void __launch_bounds__(512, 1) flash_fwd6_kernel(FaParams p) {
         const uint32_t now = (uint32_t)((j & (F6_RING - 1)) * F6_STEP);
         dma_step(j + 2, (j + 2) & (F6_RING - 1));
         const int kb = 2 * j + kh;
-        if (kb <= last) block(kb, now, j == 0);
+        if (kb <= last) block(kb, now);
         asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");   // this wavefront's part of step j + 1 landed
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
@@ -1264,8 +1269,8 @@ __global__ void __launch_bounds__(512, 1) flash_fwd6_kernel(FaParams p) {
     __syncthreads();
 
     // ---- merge.  Of its two partial results a group's wavefront kh finishes query half kh (QH = 2) or
-    // columns 32 kh .. + 31 (QH = 1) and hands over the rest; a wavefront with no block has m = -inf
-    // and weighs nothing.
+    // columns 32 kh .. + 31 (QH = 1) and hands over the rest; a wavefront with no block or no
+    // finite score has m = -inf and weighs nothing.
     constexpr int ND = QH == 2 ? 2 : 1;   // 32-column tiles this wavefront finishes
     f32x16 keep[ND];
     const int peer = w ^ 4;
@@ -1290,11 +1295,11 @@ __global__ void __launch_bounds__(512, 1) flash_fwd6_kernel(FaParams p) {
         float a, b;
         f5_xor32_pair(l_run[qh], a, b);
         l_all[qh] = a + b;
-        if (h == 0) stat[w][qh][r32] = make_float2(kh <= last ? m_run[qh] : -INFINITY, l_all[qh]);
+        if (h == 0) stat[w][qh][r32] = make_float2(m_run[qh], l_all[qh]);
     }
     __syncthreads();
     const int mq = QH == 2 ? kh : 0;
-    const float m_own = kh > last ? -INFINITY : (QH == 2 && kh ? m_run[QH - 1] : m_run[0]), l_own = QH == 2 && kh ? l_all[QH - 1] : l_all[0];
+    const float m_own = QH == 2 && kh ? m_run[QH - 1] : m_run[0], l_own = QH == 2 && kh ? l_all[QH - 1] : l_all[0];
     const float2 ot = stat[peer][mq][r32];
     const float m_all = fmaxf(m_own, ot.x);
     const float a_own = __builtin_amdgcn_exp2f(m_own - m_all), a_ot = __builtin_amdgcn_exp2f(ot.x - m_all);

@@ -47,3 +47,33 @@ def test_flash_d64_one_wavefront(gpu, E, L, H, B, scale, pad, causal):
         want = (p / p.sum(axis=1, keepdims=True)) @ v[:E, :, h, b].T.astype(np.float64)
         err = np.linalg.norm(got[:E, :, h, b].T - want) / np.linalg.norm(want)
         assert err <= 2e-3, (h, b, err)
+
+
+@pytest.mark.parametrize("causal,masked", [(True, [1]), (False, [1]), (False, [0, 1, 3]), (False, [16])])
+@pytest.mark.parametrize("E,L,H,B", [(64, 1025, 4, 1), (56, 1152, 3, 1), (64, 4160, 32, 4)])
+def test_flash_d64_infinite_scores(gpu, E, L, H, B, causal, masked):
+    """Key blocks of 64 masked by K = -inf where Q = 1: a wavefront's first block, its first two, its last (or
+    a single last key).  Every query keeps a finite score, so the result is finite and that of softmax."""
+    lh = gpu
+    announce(f"flash D={E} infinite scores S={L} H={H} B={B} causal={causal} masked={masked}")
+    rng = np.random.default_rng(E + L + masked[0])
+    q, k, v = (rng.standard_normal((E, L, 1, 1)).astype(np.float16) for _ in range(3))
+    q[0], k[0] = 1, 0
+    for m in masked:
+        k[0, 64 * m:64 * m + 64] = -np.inf
+    Q, K, V = (lh.HIPDeviceArray.from_numpy(np.asfortranarray(np.tile(t, (1, 1, H, B))), "f16") for t in (q, k, v))
+    O = lh.HIPDeviceArray("f16", (E, L, H, B))
+    lh.kernel_log_clear()
+    lh.flash_attn_fwd(O, Q, K, V, causal=causal)
+    assert lh.kernel_log()[0] == "flash_fwd6_kernel", lh.kernel_log()
+    got = O.to_numpy().astype(np.float64)
+    s = q[1:, :, 0, 0].T.astype(np.float64) @ k[1:, :, 0, 0].astype(np.float64) / math.sqrt(E)
+    for m in masked:
+        s[:, 64 * m:64 * m + 64] = -np.inf
+    if causal:
+        s = np.where(np.tril(np.ones((L, L), bool)), s, -np.inf)
+    p = np.exp(s - s.max(axis=1, keepdims=True))
+    want = (p / p.sum(axis=1, keepdims=True)) @ v[:, :, 0, 0].T.astype(np.float64)
+    for h, b in {(0, 0), (H - 1, B - 1)}:
+        err = np.linalg.norm(got[:, :, h, b].T - want) / np.linalg.norm(want)
+        assert err <= 2e-3, (h, b, err)
