@@ -290,7 +290,7 @@ def bench_vendor_bf16(steps, warmup, n=8192):
 # ---------------------------------------------------------------- CPU baseline
 def cpu_baseline_gemm(n=8192, budget_s=20.0):
     """The oracle's fp32-accumulate GEMM (a port of the tile loop, not the Lava
-    path: Julia/Mantle/lavapipe are not on the GPU box) on all host threads, over
+    path: Julia, Mantle and lavapipe are not installed) on all host threads, over
     as many rows of the same 8192^3 bf16 problem as fit the time budget (all of
     them on a 16-core host)."""
     sys.path.insert(0, str(REPO))
@@ -315,8 +315,8 @@ def cpu_baseline_gemm(n=8192, budget_s=20.0):
                       f"includes decoding B), oracle/lava_oracle.c oracle_gemm_f32acc, {dt:.1f} s"}
 
 
-# what the CPU figures are: the reference's own CPU path (Lava on lavapipe) cannot run on the box
-CPU_NOTE = ("lavapipe baseline unavailable (no Julia, Mantle or Lavapipe_jll on the GPU box); not the Lava path: "
+# what the CPU figures are: the reference's own CPU path (Lava on lavapipe) cannot run without them
+CPU_NOTE = ("lavapipe baseline unavailable (no Julia, Mantle or Lavapipe_jll installed); not the Lava path: "
             "the build's own CPU restatement (oracle/lava_oracle.c, OpenMP over all host threads)")
 
 

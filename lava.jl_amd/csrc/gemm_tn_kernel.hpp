@@ -246,7 +246,7 @@ struct TnSide<T, false, 128> {
 // M/N-contiguous int8: the slice is 128 rows of K x 256 bytes (256 m or n).  Row r's logical
 // 16-byte chunk c is stored at slot c ^ F8(r), F8(r) = (r % 8) | 8 (r / 16 % 2).  A fragment is
 // two transposing reads (ds_read_b64_tr_b8: in a 16-lane group, output lane i byte j is the
-// byte at source lane 2 j + i / 8's address + i % 8; measured on the box).  Source lane s of
+// byte at source lane 2 j + i / 8's address + i % 8; measured).  Source lane s of
 // 16-lane group g points at k row 64 u + 16 g + 8 h + s / 2 of k-step u (h = 0, 1 for the two
 // reads), byte 8 (s % 2) of the block's chunk, so output lane i receives the k-values
 // 64 u + 16 g + 8 h + [0, 8) of column 16 t + i: together the 16 k-slots a K-contiguous
