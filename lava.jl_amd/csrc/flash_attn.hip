@@ -694,8 +694,9 @@ __global__ void __launch_bounds__(128 * F5_PAIRS, 1) flash_fwd5_kernel(FaParams 
         // bias k-step: ones (key rows, k = 0) times -m (query columns, k = 0).  The
         // accumulator then holds S' = c q.k - m directly and P = exp2(S') needs no
         // per-score multiply-add.  m is kept fp16-representable for that; a rescaled block,
-        // c > 1, or a maximum beyond +-60000 (after which the wavefront stays on this path)
-        // take P = exp2(fma(S, c', -m')) in fp32 instead.
+        // c > 1, or a maximum beyond +-32768 (after which the wavefront stays on this path)
+        // take P = exp2(fma(S, c', -m')) in fp32 instead.  (Up to there m is off by at most 8, and P
+        // at most 2^8; beyond it by up to 16, and P = 2^16 is infinite in fp16.)
         const float c = p.scale_log2;
         bool fast = c <= 1.f;                    // wavefront-uniform
         if (fast) {
@@ -797,7 +798,7 @@ __global__ void __launch_bounds__(128 * F5_PAIRS, 1) flash_fwd5_kernel(FaParams 
                     // the first block sets m to its maximum (it always holds key 0, so it
                     // is never fully masked); later ones only raise it
                     mn[qh] = m_run[qh] + (first ? t[qh] : fmaxf(t[qh], 0.f));
-                    ovf = ovf || !(fabsf(mn[qh]) <= 60000.f);
+                    ovf = ovf || !(fabsf(mn[qh]) <= 32768.f);
                 }
                 if (fast && __builtin_amdgcn_ballot_w64(ovf) != 0) fast = false;
                 float alpha[QH];

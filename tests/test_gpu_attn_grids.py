@@ -59,3 +59,26 @@ def _run(lh, E, L, H, B, causal, kernel):
         want = (p / p.sum(axis=1, keepdims=True)) @ v[:, :, h, b].T.astype(np.float64)
         err = np.linalg.norm(got[:, :, h, b].T - want) / np.linalg.norm(want)
         assert err <= 2e-3, (h, b, err)
+
+
+@pytest.mark.parametrize("H,B", [(32, 16), (3, 1)])
+@pytest.mark.parametrize("low", [1.75, 0.9375])
+@pytest.mark.parametrize("E", [32, 128])
+def test_flash_scores_near_the_lowest(gpu, E, low, H, B):
+    """Every score -57328 (-30712) in base 2, halfway between two fp16 numbers 32 (16) apart: all keys weigh the
+    same, and the result is the mean of V, not what an fp16 maximum 16 below the scores would make of it."""
+    lh, L = gpu, 321
+    announce(f"flash low scores D={E} low={low} H={H} B={B}")
+    q, k = (np.zeros((E, L, H, B), np.float16, order="F") for _ in range(2))
+    q[0], k[0] = low, -65504
+    q[1], k[1] = 1, -24 if low == 1.75 else -14   # base 2: -65504 low / 2 + k[1] / 2
+    v = np.asfortranarray(np.random.default_rng(E).standard_normal((E, L, H, B)).astype(np.float16))
+    Q, K, V = (lh.HIPDeviceArray.from_numpy(t, "f16") for t in (q, k, v))
+    O = lh.HIPDeviceArray("f16", (E, L, H, B))
+    lh.kernel_log_clear()
+    lh.flash_attn_fwd_raw(Q.ptr, K.ptr, V.ptr, O.ptr, B, H, L, E, Q.strides(), O.strides(), 0.5 * math.log(2), False)
+    assert lh.kernel_log() == _kernel(E, L, H * B), lh.kernel_log()
+    got = O.to_numpy().astype(np.float64)
+    want = np.broadcast_to(v.astype(np.float64).mean(axis=1, keepdims=True), got.shape)
+    err = np.linalg.norm(got - want) / np.linalg.norm(want)
+    assert err <= 2e-3, err
